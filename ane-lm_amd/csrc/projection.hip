@@ -25,75 +25,11 @@
 
 #include <algorithm>
 
-#include "anelm_common.hpp"
+#include "projection.hpp"
 
 namespace anelm {
 
 namespace {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float r16(float v) { return (float)to_f16(v); }
-// fp16 bits (low 16 of h) widened exactly
-__device__ __forceinline__ float h2f_bits(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
-
-__device__ __forceinline__ half8 to_half8(float4 a, float4 b) {
-    half8 r;
-    r[0] = to_f16(a.x);
-    r[1] = to_f16(a.y);
-    r[2] = to_f16(a.z);
-    r[3] = to_f16(a.w);
-    r[4] = to_f16(b.x);
-    r[5] = to_f16(b.y);
-    r[6] = to_f16(b.z);
-    r[7] = to_f16(b.w);
-    return r;
-}
-
-__device__ __forceinline__ half8 as_half8(uint4 u) {
-    half8 r;
-    __builtin_memcpy(&r, &u, 16);
-    return r;
-}
-
-// (x * s) * gamma for four inputs, gamma as two packed bf16 pairs: the fused
-// RMSNorm's output, before its fp16 rounding
-__device__ __forceinline__ float4 norm_scale(float4 v, float s, uint32_t g01, uint32_t g23) {
-    v.x = (v.x * s) * bf16_to_f32(g01 & 0xFFFFu);
-    v.y = (v.y * s) * bf16_to_f32(g01 >> 16);
-    v.z = (v.z * s) * bf16_to_f32(g23 & 0xFFFFu);
-    v.w = (v.w * s) * bf16_to_f32(g23 >> 16);
-    return v;
-}
-
-struct ProjArgs {
-    float* y;
-    const void* x;  // fp32, or fp16 already rounded (XH)
-    const uint16_t* w;
-    int out_dim, in_dim, batch;
-    long ld_x, ld_y;
-    // fused prologue (kNorm): x replaced by rmsnorm(x) * gamma, gamma bf16 [in_dim]
-    const uint16_t* gamma;
-    float eps;
-    // SwiGLU epilogue (kSwiGLU, kSwiGLU16): the up rows follow the gate rows at this offset
-    long pair_rows;
-    // kSwiGLU16, kStore16: the output as fp16 bits (row stride ld_y) instead of y
-    uint16_t* y16;
-    // y rows 16-byte aligned (y and ld_y), for the LDS kernel's float4 stores
-    bool vec_y;
-};
-
-// What the epilogue does with the rounded projection p = fp16(sum) (as fp32):
-enum Epilogue {
-    kStore = 0,   // y = p
-    kAdd = 1,     // y = y + p  (the residual add of qwen3.cpp:516, :527)
-    kSwiGLU = 2,  // y = silu(p_gate) * p_up  (core/ane_runtime.cpp:393-395)
-    kSwiGLU16 = 3,  // the same rounded to fp16 (nearest even) into y16: the next projection's input
-    kStore16 = 4,   // y16 = p as fp16 bits (the ANE kernels' own fp16 output)
-    kSwiGLU16T = 5, // kSwiGLU16 with y16 in the tiled layout (out_dim columns): the tiled projection's input
-};
-constexpr bool is_swiglu(int epi) { return epi == kSwiGLU || epi == kSwiGLU16 || epi == kSwiGLU16T; }
 
 // kNorm (fp32 x): the workgroup first computes the RMSNorm scale
 // 1/sqrtf(ss/dim + eps) of each of its batch rows (core/cpu_ops.cpp:25-31),
@@ -813,10 +749,14 @@ int cu_count() {
 
 // Past 16 rows of fp16 x, against at least 8192 output rows: W streams once
 // through the LDS kernel (measured for the 151936-row LM head; narrower W is
-// better served by more, smaller workgroups).
+// better served by more, smaller workgroups), as long as one workgroup's LDS
+// holds every row of x.  More rows mean reading W again per block of them, and
+// the block-tiled kernel wins: 151936 x 1024, 64 rows 60.9 us against 69.7 (its
+// best shape), 100 rows 108 against 83; 151936 x 4096 (16 rows a workgroup), 48
+// rows 670 against 240.
 bool lds_ok(const ProjArgs& a) {
     return a.batch > 16 && a.out_dim >= 8192 && a.in_dim % 256 == 0 && a.in_dim <= 4096 && a.ld_x % 8 == 0 &&
-           aligned16(a.x) && aligned16(a.w);
+           aligned16(a.x) && aligned16(a.w) && (a.batch <= lds_rows(a.in_dim) || !gemm_takes(a, kStore));
 }
 
 template <int EPI, bool TILED = false>
@@ -871,6 +811,7 @@ template <bool XH>
 int proj_mfma(const ProjArgs& a, hipStream_t st) {
     const long tiles16 = (long)((a.out_dim + 15) / 16) * ((a.batch + 15) / 16);
     if (XH && lds_ok(a)) launch_lds<kStore>(a, st);
+    else if (XH && gemm_takes(a, kStore)) launch_gemm<kStore, false, false>(a, st);
     else if (a.batch <= 16 || tiles16 < 512) launch_mfma<XH, 1, 1, 8>(a, st);
     else launch_mfma<XH, 2, 2, XH ? 8 : 4>(a, st);
     return launch_status("proj_f16");
@@ -961,19 +902,23 @@ void f32_fused(const ProjArgs& a, hipStream_t st) {
 // The SwiGLU past 32 rows takes all 64 batch rows of a workgroup (each
 // gate|up tile read by one workgroup): 9.8 us against 11.8 us with 32 at the
 // Qwen3-0.6B shape and 64 rows; the other shapes measured no better so.
-// Shapes on fp16 x (every one 4 waves splitting the input steps, so every
-// shape gives the same bits).  Up to 16 rows: one 16-row batch block, one row
+// Shapes on fp16 x (every one here 4 waves splitting the input steps, so every
+// shape gives the same bits; each choice depends on sizes alone, so that
+// every layout of the same projection takes the same one).  Up to 16 rows: one 16-row batch block, one row
 // tile per workgroup, 8 steps of loads in flight per wave.  Past 16 rows
 // (measured at 64 rows on the Qwen3-0.6B layer shapes): the SwiGLU's gate|up
 // tile pairs take all 64 batch rows of a workgroup with 8 steps in flight;
 // shapes with many output tiles take 32 x 32 tiles; the others 16 x 16 tiles
 // with a wave's whole share of the input steps (up to 24) in flight at once.
+// With enough blocks for the chip, the block-tiled kernel (gemm.hip).
 template <int EPI, bool TILED = false, bool XT = false>
 void x16_mfma(const ProjArgs& a, hipStream_t st) {
     const long tiles16 = (long)((a.out_dim + 15) / 16) * ((a.batch + 15) / 16);
     constexpr int RT = is_swiglu(EPI) ? 2 : 1;
     const int steps = a.in_dim / 32 / 4;   // per wave
-    if (a.batch <= 16) {
+    if (gemm_takes(a, EPI)) {
+        launch_gemm<EPI, TILED, XT>(a, st);
+    } else if (a.batch <= 16) {
         launch_mfma<true, 1, RT, 8, false, EPI, 4, TILED, XT>(a, st);
     } else if constexpr (is_swiglu(EPI)) {
         if (a.batch > 32) launch_mfma<true, 4, 2, 8, false, EPI, 4, TILED, XT>(a, st);
@@ -1203,7 +1148,7 @@ extern "C" int anelm_linear_f16(uint16_t* y16, const uint16_t* x16, const uint16
     a.y16 = y16;
     hipStream_t st = as_stream(stream);
     if (lds_ok(a)) launch_lds<kStore16>(a, st);
-    else if (mfma_ok(x16, true, w16, in_dim, ld_x)) launch_mfma<true, 1, 1, 8, false, kStore16>(a, st);
+    else if (mfma_ok(x16, true, w16, in_dim, ld_x)) x16_mfma<kStore16>(a, st);
     else launch_generic<true, kStore16>(a, st);
     return launch_status("linear_f16");
 }

@@ -143,3 +143,67 @@ def test_proj_f16_tt_adjacent_buffers(hip, rng):
     hip.proj_tile_f16(xt2, xr)
     hip.proj_f16_tt(ref, xt2, wt, B, out_dim, in_dim, epilogue=hip.PROJ_STORE)
     assert_bitexact(host(y), host(ref), "adjacent y and x_t")
+
+
+# Many rows of x: the block-tiled kernel's four block shapes (chosen by the
+# number of blocks), each with a last batch block, output block and input step
+# that are only partly there: 1 (129 blocks of 32 x 128; an output count that
+# is no multiple of 4, one input step), 1 again (three input steps for two
+# groups of two), 2 (256 blocks of 64 x 128, 33 steps for four groups), 3 (320
+# blocks, odd steps), 4 (715 blocks); and fewer blocks than it takes.
+@pytest.mark.parametrize("B,out_dim,in_dim", [(65, 5501, 32), (65, 5504, 96), (17, 16352, 64), (200, 8160, 1056),
+                                               (300, 8160, 160), (700, 8288, 64), (70, 1024, 96)])
+def test_many_rows(hip, orc, rng, B, out_dim, in_dim):
+    """Every epilogue and layout: within an fp16 ulp of the oracle, tiled
+    layouts bit-identical to row-major, fp16 stores the fp32 ones narrowed."""
+    import torch
+    from test_gpu_qwen3 import _proj_ref, _ulp16, check_projection
+
+    x = (2 * rng.standard_normal((B, in_dim))).astype(np.float32)
+    x16 = orc.f32_to_f16_rne(x).reshape(B, in_dim)
+    w = (0.03 * rng.standard_normal((out_dim, in_dim))).astype(np.float16).view(np.uint16)
+    xr, dw = dev(x16.view(np.int16)), dev(w.view(np.int16))
+    xt, wt = tiled_buf(B, in_dim), tiled_buf(out_dim, in_dim)
+    hip.proj_tile_f16(xt, xr)
+    hip.proj_tile_f16(wt, dw)
+
+    def three(n, epi, dt, y0=None):
+        """The output of the row-major call, checked against the two tiled ones."""
+        ys = [dev(y0) if y0 is not None else torch.full((B, n), -1, dtype=dt, device="cuda") for _ in range(3)]
+        if epi != hip.PROJ_STORE_F16:
+            hip.proj_f16_x16_fused(ys[0], xr, dw, epilogue=epi)
+        else:
+            hip.linear_f16(ys[0], xr, dw)
+        hip.proj_f16_x16_tiled(ys[1], xr, wt, n, epilogue=epi)
+        hip.proj_f16_tt(ys[2], xt, wt, B, n, in_dim, epilogue=epi)
+        for y in ys[1:]:
+            assert_bitexact(host(y), host(ys[0]), f"layouts, epilogue {epi}")
+        return host(ys[0])
+
+    y = three(out_dim, hip.PROJ_STORE, torch.float32)
+    check_projection(orc, x, w, y.astype(np.float64))
+    y2 = torch.full((B, out_dim), -1.0, device="cuda")
+    hip.proj_f16_x16(y2, xr, dw)
+    assert_bitexact(host(y2), y, "proj_f16_x16")
+    y16 = three(out_dim, hip.PROJ_STORE_F16, torch.int16)
+    assert_bitexact(y16, orc.f32_to_f16_rne(y).reshape(B, out_dim).view(np.int16), "fp16 store")
+    r0 = rng.standard_normal((B, out_dim)).astype(np.float32)
+    assert_bitexact(three(out_dim, hip.PROJ_ADD, torch.float32, r0), r0 + y, "residual add")
+    # one float off a 16-byte boundary: the element-wise stores
+    off = torch.full((B * out_dim + 1,), -1.0, device="cuda")
+    hip.proj_f16_x16_fused(off[1:].view(B, out_dim), xr, dw)
+    assert_bitexact(host(off[1:].view(B, out_dim)), y, "unaligned output")
+    if out_dim % 32 == 0:
+        n = out_dim // 2
+        h = three(n, hip.PROJ_SWIGLU, torch.float32)
+        g, u = y[:, :n].astype(np.float64), y[:, n:].astype(np.float64)
+        want = g / (1 + np.exp(-g)) * u
+        assert np.all(np.abs(h - want) <= 1e-5 * np.abs(want) + 1e-30)
+        h16 = three(n, hip.PROJ_SWIGLU_F16, torch.int16)
+        assert_bitexact(h16, orc.f32_to_f16_rne(h).reshape(B, n).view(np.int16), "fp16 SwiGLU")
+        if n % 32 == 0:
+            ht = tiled_buf(B, n)
+            hip.proj_f16_tt(ht, xt, wt, B, n, in_dim, epilogue=hip.PROJ_SWIGLU_F16_TILED)
+            assert_bitexact(untile(host(ht), B, n), h16, "tiled fp16 SwiGLU")
+            pad = np.asarray(host(ht)).reshape((B + 15) // 16, n // 32, 4, 16, 8)[-1, :, :, (B - 1) % 16 + 1:]
+            assert np.all(pad.astype(np.uint16) == 0xFFFF), "rows past the batch are left as they are"
