@@ -34,6 +34,7 @@ SOURCES = [
     os.path.join(CSRC, "attention.hip"),
     os.path.join(CSRC, "deltanet.hip"),
     os.path.join(CSRC, "projection.hip"),
+    os.path.join(CSRC, "rows.hip"),
     os.path.join(CSRC, "gemm.hip"),
     os.path.join(HOST, "dropin.hip"),
     os.path.join(HOST, "safetensors.hip"),

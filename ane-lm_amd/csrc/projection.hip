@@ -19,6 +19,8 @@
 // the partials behind a device-scope fence, measured 20 us slower per call:
 // the fence writes back the L2.)
 //
+// 3 to 16 rows against a row-major W: rows.hip.  Many rows: gemm.hip.
+//
 // Dot path (one or two rows of x, up to eight for narrow out_dim; in_dim any
 // multiple of 8): one wave per output row, v_dot2_f32_f16 into fp32.
 #include <hip/hip_runtime.h>
@@ -458,15 +460,6 @@ __device__ __forceinline__ half2v as_half2(uint32_t u) {
     return r;
 }
 
-__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, to_f16(lo)) | ((uint32_t)__builtin_bit_cast(uint16_t, to_f16(hi)) << 16);
-}
-
-enum : int {
-    kXF32 = 0,
-    kXNorm = 1,
-    kXF16 = 2,
-};
 constexpr int kDotNormMaxIn = 4096;   // kXNorm: LDS for the staged rows (8 KB per row of x)
 
 // kXNorm: 4-input slices per thread that cover in_dim for a chunk count
@@ -672,10 +665,16 @@ void proj_dot(const ProjArgs& a, hipStream_t st) {
     else dot_shape<8, XM, EPI>(a, st);
 }
 
-// Where the dot kernel beats the MFMA kernel (measured at the Qwen3-0.6B
-// decode shapes): one or two rows of x everywhere, up to eight for narrow
-// out_dim (1024 rows: 64 MFMA workgroups).
-bool dot_wins(long batch, int out_dim) { return batch <= 2 || (batch <= 8 && out_dim <= 1024); }
+// Where the dot kernel beats the MFMA kernels: one or two rows of x (gate|up
+// of 2560 x 9728, 2 rows: 19.1 us against 24.1 in rows.hip), but, without a
+// norm or a SwiGLU (plain), not two rows of 4096 or more inputs into 2560 or more outputs, which it takes in
+// several rounds of loads (2560 x 9728 down: 15.1 against 12.3); and up to
+// eight for narrow out_dim and short rows (3 rows, 1024 x 2048: 3.5 against
+// 3.9; 5 rows, 896 x 4864: 8.3 against 5.8).
+bool dot_wins(long batch, int out_dim, int in_dim, bool plain) {
+    if (batch == 2 && plain && in_dim >= 4096 && out_dim >= 2560) return false;
+    return batch <= 2 || (batch <= 8 && out_dim <= 1024 && in_dim <= 3072);
+}
 
 // y and x must not share memory: workgroups write y while others still read x.
 bool overlaps(const void* y, long ld_y, int out_dim, int y_bytes, const void* x, long ld_x, int in_dim, int x_bytes,
@@ -799,11 +798,9 @@ void launch_mfma(const ProjArgs& a, hipStream_t st) {
     proj_mfma_kernel<XH, NB, RT, R, NORM, EPI, NW, TILED, XT><<<grid, dim3(64 * NW), 0, st>>>(a);
 }
 
-// Up to 16 rows: one 16-row batch block, one row tile per workgroup (the
-// most workgroups), 8 steps of loads in flight per wave.  Past 16 rows,
-// 32-row batch blocks with two row tiles per workgroup (each input fetched
-// from cache feeds four MFMA tiles) where that still leaves enough
-// workgroups; shapes with few output tiles (out_dim 1024 at 64 rows: 64 such
+// Up to 16 rows: rows.hip.  Past 16 rows, 32-row batch blocks with two row
+// tiles per workgroup (each input fetched from cache feeds four MFMA tiles)
+// where that still leaves enough workgroups; shapes with few output tiles (out_dim 1024 at 64 rows: 64 such
 // workgroups) keep 16x16 tiles and four times the workgroups, which measured
 // 1.6x faster there.  (8 waves per workgroup for the few-tile shapes
 // measured 10% slower than 4.)
@@ -811,6 +808,7 @@ template <bool XH>
 int proj_mfma(const ProjArgs& a, hipStream_t st) {
     const long tiles16 = (long)((a.out_dim + 15) / 16) * ((a.batch + 15) / 16);
     if (XH && lds_ok(a)) launch_lds<kStore>(a, st);
+    else if (rows_takes(a)) launch_rows<XH ? kXF16 : kXF32, kStore>(a, st);
     else if (XH && gemm_takes(a, kStore)) launch_gemm<kStore, false, false>(a, st);
     else if (a.batch <= 16 || tiles16 < 512) launch_mfma<XH, 1, 1, 8>(a, st);
     else launch_mfma<XH, 2, 2, XH ? 8 : 4>(a, st);
@@ -858,7 +856,7 @@ extern "C" int anelm_proj_f16(float* y, const float* x, const uint16_t* w16, lon
     hipStream_t st = as_stream(stream);
     const ProjArgs a = args(y, x, w16, batch, out_dim, in_dim, ld_x, ld_y);
     const bool dot = dot_ok(x, w16, batch, in_dim, ld_x);
-    if (mfma_ok(x, false, w16, in_dim, ld_x) && !(dot && dot_wins(batch, out_dim))) return proj_mfma<false>(a, st);
+    if (mfma_ok(x, false, w16, in_dim, ld_x) && !(dot && dot_wins(batch, out_dim, in_dim, true))) return proj_mfma<false>(a, st);
     if (dot) {
         proj_dot<kXF32, kStore>(a, st);
     } else {
@@ -884,14 +882,15 @@ extern "C" int anelm_proj_f16_x16(float* y, const uint16_t* x16, const uint16_t*
     return proj_mfma<true>(args(y, x16, w16, batch, out_dim, in_dim, ld_x, ld_y), as_stream(stream));
 }
 
-// fp32 inputs with the fused RMSNorm and epilogues: one 16-row batch block
-// per workgroup up to 16 rows, and past that wherever there are few output
-// tiles; otherwise 32-row batch blocks and two row tiles per workgroup.
+// fp32 inputs with the fused RMSNorm and epilogues: rows.hip up to 16 rows;
+// past that one 16-row batch block per workgroup wherever there are few output
+// tiles, otherwise 32-row batch blocks and two row tiles per workgroup.
 template <bool NORM, int EPI>
 void f32_fused(const ProjArgs& a, hipStream_t st) {
     const long tiles16 = (long)((a.out_dim + 15) / 16) * ((a.batch + 15) / 16);
     constexpr int RT = is_swiglu(EPI) ? 2 : 1;
-    if (a.batch <= 16 || (!is_swiglu(EPI) && tiles16 < 512)) launch_mfma<false, 1, RT, 8, NORM, EPI>(a, st);
+    if (rows_takes(a)) launch_rows<NORM ? kXNorm : kXF32, EPI>(a, st);
+    else if (a.batch <= 16 || (!is_swiglu(EPI) && tiles16 < 512)) launch_mfma<false, 1, RT, 8, NORM, EPI>(a, st);
     else launch_mfma<false, 2, 2, 4, NORM, EPI>(a, st);
 }
 
@@ -904,9 +903,9 @@ void f32_fused(const ProjArgs& a, hipStream_t st) {
 // Qwen3-0.6B shape and 64 rows; the other shapes measured no better so.
 // Shapes on fp16 x (every one here 4 waves splitting the input steps, so every
 // shape gives the same bits; each choice depends on sizes alone, so that
-// every layout of the same projection takes the same one).  Up to 16 rows: one 16-row batch block, one row
-// tile per workgroup, 8 steps of loads in flight per wave.  Past 16 rows
-// (measured at 64 rows on the Qwen3-0.6B layer shapes): the SwiGLU's gate|up
+// every layout of the same projection takes the same one).  Up to 16 rows (W
+// tiled): one 16-row batch block, one row tile per workgroup, 8 steps of loads
+// in flight per wave.  Past 16 rows (measured at 64 rows on the Qwen3-0.6B layer shapes): the SwiGLU's gate|up
 // tile pairs take all 64 batch rows of a workgroup with 8 steps in flight;
 // shapes with many output tiles take 32 x 32 tiles; the others 16 x 16 tiles
 // with a wave's whole share of the input steps (up to 24) in flight at once.
@@ -933,8 +932,9 @@ void x16_mfma(const ProjArgs& a, hipStream_t st) {
 
 template <int EPI>
 void x16_fused(const ProjArgs& a, hipStream_t st) {
-    if (dot16_ok(static_cast<const uint16_t*>(a.x), a.w, a.batch, a.in_dim, a.ld_x) && dot_wins(a.batch, a.out_dim))
+    if (dot16_ok(static_cast<const uint16_t*>(a.x), a.w, a.batch, a.in_dim, a.ld_x) && dot_wins(a.batch, a.out_dim, a.in_dim, !is_swiglu(EPI)))
         proj_dot<kXF16, EPI>(a, st);
+    else if (rows_takes(a)) launch_rows<kXF16, EPI>(a, st);
     else if (EPI == kStore && lds_ok(a)) launch_lds<kStore>(a, st);
     else x16_mfma<EPI>(a, st);
 }
@@ -1092,7 +1092,8 @@ extern "C" int anelm_proj_f16_fused(void* y, const float* x, const uint16_t* w16
     a.pair_rows = out_dim;  // SwiGLU: W holds out_dim gate rows, then out_dim up rows
     hipStream_t st = as_stream(stream);
     const bool norm = norm_bf16 != nullptr;
-    if (dot_ok(x, w16, batch, in_dim, ld_x) && dot_wins(batch, out_dim) && (!norm || in_dim <= kDotNormMaxIn)) {
+    const bool plain = !norm && epilogue <= ANELM_PROJ_ADD;
+    if (dot_ok(x, w16, batch, in_dim, ld_x) && dot_wins(batch, out_dim, in_dim, plain) && (!norm || in_dim <= kDotNormMaxIn)) {
         switch (epilogue) {
             case ANELM_PROJ_STORE:
                 if (norm) proj_dot<kXNorm, kStore>(a, st);
@@ -1148,6 +1149,7 @@ extern "C" int anelm_linear_f16(uint16_t* y16, const uint16_t* x16, const uint16
     a.y16 = y16;
     hipStream_t st = as_stream(stream);
     if (lds_ok(a)) launch_lds<kStore16>(a, st);
+    else if (mfma_ok(x16, true, w16, in_dim, ld_x) && rows_takes(a)) launch_rows<kXF16, kStore16>(a, st);
     else if (mfma_ok(x16, true, w16, in_dim, ld_x)) x16_mfma<kStore16>(a, st);
     else launch_generic<true, kStore16>(a, st);
     return launch_status("linear_f16");

@@ -70,6 +70,22 @@ enum Epilogue {
 };
 constexpr bool is_swiglu(int epi) { return epi == kSwiGLU || epi == kSwiGLU16 || epi == kSwiGLU16T; }
 
+__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
+    return (uint32_t)__builtin_bit_cast(uint16_t, to_f16(lo)) | ((uint32_t)__builtin_bit_cast(uint16_t, to_f16(hi)) << 16);
+}
+
+// the forms of x (see proj_dot_kernel)
+enum : int {
+    kXF32 = 0,
+    kXNorm = 1,
+    kXF16 = 2,
+};
+
+// ---- 3 to 16 rows of x, W row-major (rows.hip)
+bool rows_takes(const ProjArgs& a);
+template <int XM, int EPI>
+void launch_rows(const ProjArgs& a, hipStream_t st);
+
 // ---- many rows of x (gemm.hip) -------------------------------------------------
 // Whether the block-tiled kernel takes a projection of fp16 x.
 bool gemm_takes(const ProjArgs& a, int epi);
