@@ -14,6 +14,9 @@
 //            K row; dots for all group heads, reduced in-row with DPP;
 //   phase 2: chunk softmax numerators (max, exp, sum) in LDS;
 //   phase 3: the same position mapping over V rows, weighted accumulation.
+// With the q/k norm + RoPE inside, each q head is made once per workgroup and
+// shared through LDS (every 16-lane group making all of them itself cost 0.4
+// us a launch and two waves per SIMD).
 // With one chunk per sequence the workgroup writes the normalised output;
 // otherwise each chunk writes (max, sum, unnormalised output) partials and
 // counts itself done, and the last chunk of a (sequence, kv head) to finish
@@ -28,8 +31,6 @@
 namespace anelm {
 namespace {
 
-constexpr int kAttnThreads = 256;     // 4 waves
-constexpr int kAttnWaves = kAttnThreads / kWave;
 constexpr int kMaxChunk = 512;        // ring positions per workgroup of a split launch
 // Whole-ring launches: with at least kWholeRingPairs (sequence, kv head)
 // pairs (two per CU) and rings of at most kWholeRingMax rows, one workgroup
@@ -40,12 +41,9 @@ constexpr int kMaxChunk = 512;        // ring positions per workgroup of a split
 // pairs per CU some CUs would run two rings and others one.
 constexpr int kWholeRingMax = 2048;
 constexpr long kWholeRingPairs = 512;
-// 64, not 32: a workgroup keeps two 32-position batches of loads in flight,
-// so a 64-position chunk costs about one memory round trip like a 32-position
-// one, and a long ring at a small batch has half the chunks to merge.
 constexpr int kMinChunk = 64;
 constexpr int kMaxGD = 1024;          // group heads x head_dim per workgroup
-constexpr long kTargetBlocks = 2048;  // 8 workgroups per CU on 256 CUs
+constexpr long kTargetBlocks = 384;   // workgroups of a split launch (see pick_chunk)
 constexpr int kMaxSplit = 4096;       // chunks per sequence (capacity <= 4096*32)
 constexpr int kWholeRows = 128;       // rings up to this long (or one chunk) are done by one workgroup
 static_assert(kWholeRows <= kMaxChunk, "a whole ring's scores fit the LDS rows");
@@ -88,6 +86,7 @@ struct AttnArgs {
     int tab_len;
     float eps;
     float inv[64];              // RoPE inverse frequencies of the 64 pairs
+    int waves;                  // waves per workgroup: 4 or 8
     int whole_ring;             // launch one workgroup per (sequence, kv head) over the whole ring
 };
 
@@ -169,7 +168,10 @@ __device__ __forceinline__ float ld_dev(const float* p) {
 // contributes nothing; NaN sums propagate.
 template <int D>
 __device__ void merge_head(const AttnArgs& a, long b, int h, int lane, int live) {
-    constexpr int kBatch = D <= 128 ? 32 : 16;  // chunks whose partials are in flight at once
+    // Chunks whose partials are in flight at once: 32 held 64 more registers
+    // through the whole kernel (3 waves per SIMD instead of 5) for a merge that
+    // pick_chunk keeps to a few batches (16 x 1024 ragged rows 26.9 -> 24.6 us).
+    constexpr int kBatch = 8;
     const int ns = a.nsplit;
     const float* p = a.ws + (b * a.nh + h) * ns * (long)(D + 2);
     auto clampc = [&](int s) { return s < live ? s : live - 1; };
@@ -231,17 +233,55 @@ __device__ void merge_head(const AttnArgs& a, long b, int h, int lane, int live)
 template <int D>
 __device__ __forceinline__ int elem_of(int ds, int i) { return (i < 4 ? 0 : D / 2 - 4) + 4 * ds + i; }
 
-template <int D, int GM, bool FINAL, int QK = -1, int MC = kMaxChunk>   // MC: chunk positions whose scores fit in LDS
-__global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
+// v0 and v1 summed over the two halves of every 2*H lanes in one add: the
+// swap puts v0's halves into the first half of the lanes of the two results
+// and v1's into the second, which then hold v0's and v1's sums.
+template <int H>
+__device__ __forceinline__ float swap_add(float v0, float v1) {
+    if constexpr (H == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v0), __float_as_uint(v1), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v0), __float_as_uint(v1), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+}
+
+// Sums acc[g][i] over the wave's groups of D/8 lanes (its position slots) and
+// hands each sum to put(g, i, sum) in the lanes of one 16-lane row (D 256: two
+// rows): a quarter of the steps of summing every element in every lane, and
+// no LDS permutes.
+template <int D, int GM, typename F>
+__device__ __forceinline__ void reduce_slots(float (&acc)[GM][8], int lane, F put) {
+    const int r = lane >> 4;
+#pragma unroll
+    for (int g = 0; g < GM; g++) {
+        if constexpr (D == 256) {
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) put(g, i + (r >> 1), swap_add<32>(acc[g][i], acc[g][i + 1]));
+        } else {
+            if constexpr (D == 64) {   // the two slots of a row first
+#pragma unroll
+                for (int i = 0; i < 8; i++) acc[g][i] += dpp<0x128>(acc[g][i]);   // row_ror 8
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i += 4)
+                put(g, i + r, swap_add<32>(swap_add<16>(acc[g][i], acc[g][i + 1]),
+                                           swap_add<16>(acc[g][i + 2], acc[g][i + 3])));
+        }
+    }
+}
+
+template <int D, int GM, bool FINAL, int QK, int MC, int W>   // MC: chunk positions whose scores fit in LDS
+__global__ __launch_bounds__(kWave* W) void gqa_decode_kernel(AttnArgs a) {
     static_assert(QK < 0 || D == 128, "the fused q/k norm + RoPE is for 128-wide heads");
     constexpr int LP = D / 8;                  // lanes per position
     constexpr int PPW = kWave / LP;            // positions per wave per round
-    constexpr int PPB = PPW * kAttnWaves;      // positions per workgroup per round
     constexpr int U = 2;                       // rounds per batch of loads (two batches in flight)
-    constexpr int STEP = U * PPB;              // positions per batch
     __shared__ float sc[GM][MC];               // scores, then weights
-    __shared__ float red[kAttnWaves][GM][D];   // per-wave partial outputs
+    __shared__ float red[W][GM][D];   // per-wave partial outputs
     __shared__ float hm[GM], hl[GM];
+    __shared__ __align__(16) float s_head[QK >= 0 ? GM + 2 : 1][D];   // QK: the q heads made here, then k and v of the new row
 
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
     const int kvh = blockIdx.x, split = blockIdx.z;
@@ -259,6 +299,12 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
     const int t0 = split * a.chunk;
     const int n = whole ? len : min(t0 + a.chunk, len) - t0;     // positions of this chunk
     if (!fin && n <= 0) return;   // past the ring: neither partials nor a count
+    // a chunk that four waves take in one batch is left to them: the others'
+    // share of the set-up and of the barriers costs more than they would save
+    const int nw = W > 4 && n <= 4 * PPW * U ? 4 : W;
+    if (wid >= nw) return;
+    const int PPB = PPW * nw;                      // positions per workgroup per round
+    const int STEP = U * PPB;                      // positions per batch
     const int ps = wid * PPW + lane / LP;          // position slot within a round
     const int ds = lane % LP;                      // this lane's 8-float slice
     const int row = a.nkv * D;                     // cap * row < 2^31 (checked on the host)
@@ -271,43 +317,45 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
     // registers: the next batch's loads are in flight while this one is
     // used.  Positions past the chunk re-read its last row (n >= 1 inside
     // the loops) and are discarded.
-    // QK: the newest row (position len-1) is made here, in this lane's slice
-    // layout, by the workgroup whose chunk holds it, substituted for what the
-    // caches held at its slot, and written to the caches once made.  The
-    // RoPE angles, gammas, raw k and v, the q heads and the first K batch are
-    // all loaded before any of them is used, so the loads overlap.
-    float knew[8], vnew[8], kr[8];
-    float4 rc, rs, gql, gqh, gkl, gkh;   // cos/sin of this lane's four angles; q and k gammas
-    const int tnew = QK >= 0 ? len - 1 - t0 : -1;   // its position in this chunk
-    const bool owns = QK >= 0 && tnew >= 0 && tnew < n;
-    // The loads are unconditional (a branch around a load makes the wave
+    // QK: each q head is normalised and rotated by one 16-lane group of the
+    // workgroup and handed to the others through LDS; the next two groups
+    // make the newest row (position len-1) from k and v, for the workgroup
+    // whose chunk holds it: it stands in for what the caches held at its slot
+    // and is written to them.  The raw row, its gamma, the RoPE angles and the
+    // first K batch are all loaded before any of them is used, so the loads
+    // overlap, and unconditionally (a branch around a load makes the wave
     // wait for it at the branch's end): a table row (the clamped position's;
-    // replaced below when the position is past the table), both gammas (non-
-    // null, checked on the host), and the raw k and v of every workgroup.
+    // replaced below when the position is past the table), and k for the
+    // groups with nothing to make.
+    const int tnew = QK >= 0 ? len - 1 - t0 : -1;   // the newest row's position in this chunk
+    const bool owns = QK >= 0 && tnew >= 0 && tnew < n;
+    const int grp = tid / LP;
+    float raw[8];
+    float4 rc, rs, gl, gh;   // cos/sin of this lane's four angles; its gammas
     const int rpos = QK >= 0 ? min(max(qpos, 0), a.tab_len - 1) : 0;   // tab_len >= 1
     if constexpr (QK >= 0) {
         constexpr int WT = QK < 0 ? ANELM_F32 : QK;
+        static_assert(4 * PPW >= GM + 2, "a group per q head, k and v");
+        const float* src = grp < gc ? a.q + b * a.q_ld + (long)(kvh * a.groups + a.g0 + grp) * a.q_hs
+                                    : (grp == gc + 1 ? a.vraw + b * a.v_ld : a.kraw + b * a.k_ld) + (long)kvh * D;
+        load8<D, false>(raw, src + 4 * ds);
+        const void* gw = grp < gc ? a.wq : a.wk;
+        gl = load_w4<WT>(gw, 4 * ds);
+        gh = load_w4<WT>(gw, 4 * ds + 64);
         rc = *reinterpret_cast<const float4*>(a.cos_tab + (long)rpos * 64 + 4 * ds);
         rs = *reinterpret_cast<const float4*>(a.sin_tab + (long)rpos * 64 + 4 * ds);
-        gql = load_w4<WT>(a.wq, 4 * ds);
-        gqh = load_w4<WT>(a.wq, 4 * ds + 64);
-        gkl = load_w4<WT>(a.wk, 4 * ds);
-        gkh = load_w4<WT>(a.wk, 4 * ds + 64);
-        load8<D, false>(kr, a.kraw + b * a.k_ld + (long)kvh * D + 4 * ds);
-        load8<D, false>(vnew, a.vraw + b * a.v_ld + (long)kvh * D + 4 * ds);
     }
     auto load_batch = [&](float (&buf)[U][8], const float* base, int r0) {
 #pragma unroll
         for (int u = 0; u < U; u++) load8<D, true>(buf[u], base + ring_slot(a, start, t0, r0 + u * PPB + ps, n) * row);
     };
-    // the newest row in place of the slot's old contents (K: knew, V: vnew)
-    auto fix_batch = [&](float (&buf)[U][8], const float (&nw)[8], int r0) {
+    // the newest row (LDS row r) in place of the slot's old contents
+    auto fix_batch = [&](float (&buf)[U][8], int r, int r0) {
         if constexpr (QK >= 0) {
+            if (owns && tnew >= r0 && tnew < r0 + STEP) {   // uniform
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const bool hit = owns && r0 + u * PPB + ps == tnew;
-#pragma unroll
-                for (int i = 0; i < 8; i++) buf[u][i] = hit ? nw[i] : buf[u][i];
+                for (int u = 0; u < U; u++)
+                    if (r0 + u * PPB + ps == tnew) load8<D, false>(buf[u], &s_head[r][4 * ds]);
             }
         }
     };
@@ -315,19 +363,18 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
     // phase 1: scores
     {
         float qv[GM][8];
+        float ka[U][8], kb[U][8];
+        if constexpr (QK < 0) {
 #pragma unroll
-        for (int g = 0; g < GM; g++) {
-            if constexpr (QK >= 0) {   // branch-free: heads past gc re-read the last one, then zeroed
-                const int gg = g < gc ? g : gc - 1;
-                load8<D, false>(qv[g], a.q + b * a.q_ld + (long)(kvh * a.groups + a.g0 + gg) * a.q_hs + 4 * ds);
-            } else if (g < gc) {
-                load8<D, false>(qv[g], a.q + b * a.q_ld + (long)(kvh * a.groups + a.g0 + g) * a.q_hs + 4 * ds);
-            } else {
+            for (int g = 0; g < GM; g++) {
+                if (g < gc) {
+                    load8<D, false>(qv[g], a.q + b * a.q_ld + (long)(kvh * a.groups + a.g0 + g) * a.q_hs + 4 * ds);
+                } else {
 #pragma unroll
-                for (int i = 0; i < 8; i++) qv[g][i] = 0.0f;
+                    for (int i = 0; i < 8; i++) qv[g][i] = 0.0f;
+                }
             }
         }
-        float ka[U][8], kb[U][8];
         if (n > 0) load_batch(ka, kbase, 0);
         if constexpr (QK >= 0) {
             if (qpos != rpos) {   // past the table (uniform): the angles themselves
@@ -336,35 +383,27 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
                 rc = fc;
                 rs = fs;
             }
-            // the q heads' norm + RoPE, every lane of each 16-lane group
-#pragma unroll
-            for (int g = 0; g < GM; g++) {
-                float4 ol, oh;
-                norm_rope128_w(make_float4(qv[g][0], qv[g][1], qv[g][2], qv[g][3]),
-                               make_float4(qv[g][4], qv[g][5], qv[g][6], qv[g][7]), true, gql, gqh, rc, rs, a.eps,
-                               ol, oh);
-                if (g >= gc) ol = oh = make_float4(0.f, 0.f, 0.f, 0.f);   // heads past gc
-                qv[g][0] = ol.x; qv[g][1] = ol.y; qv[g][2] = ol.z; qv[g][3] = ol.w;
-                qv[g][4] = oh.x; qv[g][5] = oh.y; qv[g][6] = oh.z; qv[g][7] = oh.w;
-            }
-            if (owns) {   // uniform across the workgroup
-                float4 ol, oh;
-                norm_rope128_w(make_float4(kr[0], kr[1], kr[2], kr[3]), make_float4(kr[4], kr[5], kr[6], kr[7]), true,
-                               gkl, gkh, rc, rs, a.eps, ol, oh);
-                knew[0] = ol.x; knew[1] = ol.y; knew[2] = ol.z; knew[3] = ol.w;
-                knew[4] = oh.x; knew[5] = oh.y; knew[6] = oh.z; knew[7] = oh.w;
+            if (grp < gc + 2) {
+                float4 ol = make_float4(raw[0], raw[1], raw[2], raw[3]), oh = make_float4(raw[4], raw[5], raw[6], raw[7]);
+                if (grp < gc + 1) norm_rope128_w(ol, oh, true, gl, gh, rc, rs, a.eps, ol, oh);
+                *reinterpret_cast<float4*>(&s_head[grp][4 * ds]) = ol;
+                *reinterpret_cast<float4*>(&s_head[grp][4 * ds + D / 2]) = oh;
                 // The new row goes to the caches now, not behind the
                 // outputs: this workgroup's own loads of its slot (the only
-                // ones) are replaced by these registers whatever they return.
-                if (tid < LP) {   // one 16-lane group stores the row
-                    const long slot = ring_slot(a, start, t0, tnew, n);
-                    float* kd = const_cast<float*>(kbase) + slot * row;
-                    float* vd = const_cast<float*>(vbase) + slot * row;
-                    *reinterpret_cast<float4*>(kd) = ol;
-                    *reinterpret_cast<float4*>(kd + D / 2) = oh;
-                    *reinterpret_cast<float4*>(vd) = make_float4(vnew[0], vnew[1], vnew[2], vnew[3]);
-                    *reinterpret_cast<float4*>(vd + D / 2) = make_float4(vnew[4], vnew[5], vnew[6], vnew[7]);
+                // ones) are replaced whatever they return.
+                if (grp >= gc && owns) {
+                    float* dst = const_cast<float*>(grp == gc ? kbase : vbase) + (long)ring_slot(a, start, t0, tnew, n) * row;
+                    *reinterpret_cast<float4*>(dst) = ol;
+                    *reinterpret_cast<float4*>(dst + D / 2) = oh;
                 }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int g = 0; g < GM; g++) {
+                load8<D, false>(qv[g], &s_head[g < gc ? g : 0][4 * ds]);
+                if (g >= gc)
+#pragma unroll
+                    for (int i = 0; i < 8; i++) qv[g][i] = 0.0f;
             }
         }
         auto scores = [&](const float (&kx)[U][8], int r0) {
@@ -385,11 +424,11 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
         };
         for (int r0 = 0; r0 < n; r0 += 2 * STEP) {
             if (r0 + STEP < n) load_batch(kb, kbase, r0 + STEP);
-            fix_batch(ka, knew, r0);
+            fix_batch(ka, gc, r0);
             scores(ka, r0);
             if (r0 + STEP >= n) break;
             if (r0 + 2 * STEP < n) load_batch(ka, kbase, r0 + 2 * STEP);
-            fix_batch(kb, knew, r0 + STEP);
+            fix_batch(kb, gc, r0 + STEP);
             scores(kb, r0 + STEP);
         }
     }
@@ -399,7 +438,7 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
     __syncthreads();
 
     // phase 2: softmax numerators per head over the chunk
-    for (int g = wid; g < gc; g += kAttnWaves) {
+    for (int g = wid; g < gc; g += nw) {
         float m = -INFINITY;
         for (int i = lane; i < n; i += kWave) m = fmaxf(m, sc[g][i]);
         m = wave_max_rows(m);
@@ -445,32 +484,20 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
     };
     for (int r0 = 0; r0 < n; r0 += 2 * STEP) {
         if (r0 + STEP < n) load_batch(vb, vbase, r0 + STEP);
-        fix_batch(va, vnew, r0);
+        fix_batch(va, gc + 1, r0);
         accumulate(va, r0);
         if (r0 + STEP >= n) break;
         if (r0 + 2 * STEP < n) load_batch(va, vbase, r0 + 2 * STEP);
-        fix_batch(vb, vnew, r0 + STEP);
+        fix_batch(vb, gc + 1, r0 + STEP);
         accumulate(vb, r0 + STEP);
     }
     // reduce over the position slots of the wave (lanes with the same slice)
-#pragma unroll
-    for (int g = 0; g < GM; g++)
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-#pragma unroll
-            for (int o = LP; o < kWave; o <<= 1) acc[g][i] += __shfl_xor(acc[g][i], o);
-    if (lane < LP) {
-#pragma unroll
-        for (int g = 0; g < GM; g++)
-#pragma unroll
-            for (int i = 0; i < 8; i++) red[wid][g][elem_of<D>(ds, i)] = acc[g][i];
-    }
+    reduce_slots<D, GM>(acc, lane, [&](int g, int i, float v) { red[wid][g][elem_of<D>(ds, i)] = v; });
     __syncthreads();
-    for (int j = tid; j < gc * D; j += kAttnThreads) {
+    for (int j = tid; j < gc * D; j += kWave * nw) {
         const int g = j / D, d = j % D;
         float s = red[0][g][d];
-#pragma unroll
-        for (int w = 1; w < kAttnWaves; w++) s += red[w][g][d];
+        for (int w = 1; w < nw; w++) s += red[w][g][d];
         const int h = kvh * a.groups + a.g0 + g;
         if (fin) {
             put_out(a, b, h * D + d, s);
@@ -506,7 +533,7 @@ __global__ __launch_bounds__(kAttnThreads) void gqa_decode_kernel(AttnArgs a) {
         }
         __syncthreads();
         if (!s_last) return;
-        for (int g = wid; g < gc; g += kAttnWaves) merge_head<D>(a, b, kvh * a.groups + a.g0 + g, lane, live);
+        for (int g = wid; g < gc; g += nw) merge_head<D>(a, b, kvh * a.groups + a.g0 + g, lane, live);
     }
 }
 
@@ -546,36 +573,67 @@ __global__ __launch_bounds__(256) void kv_ring_advance_kernel(int32_t* rs, int32
     ring_advance(rs + r, rl + r, cap);
 }
 
-// Positions per workgroup for a ring of `bound` positions and `pairs`
-// (sequence, kv head) pairs: the largest chunk that still gives about
-// kTargetBlocks workgroups, at least kMinChunk.
-int pick_chunk(long pairs, int bound) {
+// Positions per workgroup for rings of `cap` positions and `pairs` (sequence,
+// kv head) pairs.  A split ring costs its last workgroup three more memory
+// round trips (partials stored, counted, read back: 2 us), and merging them
+// takes longer the more there are; a CU pulls a ring in at no more than about
+// 45 GB/s, whatever its waves, so few workgroups are slow too.  The largest
+// chunk that gives kTargetBlocks workgroups; below that 64 positions (128 for
+// rings of more than 16 such chunks); and rings of up to 256 rows are not
+// split at all once half the CUs have one.  us per launch with chunks of
+// 64 / 128 / 256 / 512 (8 waves, 8 kv heads, fused q/k norm):
+//     1 sequence  x  512 rows:   7.8 /  9.3 / 12.4 / 16.7
+//     1 sequence  x 2048 rows:  12.6 / 11.8 / 14.1 / 20.9
+//     8 sequences x 1024 rows:  18.2 / 13.5 / 15.0 / 21.5   (ragged lengths)
+//    16 sequences x 1024 rows:  27.2 / 23.2 / 20.1 / 23.1   (ragged lengths)
+//    48 sequences x 2048 rows: 115   / 93   / 82   / 79     (ragged lengths)
+//    20 sequences x  256 rows:  15.3 / 13.9 / 12.5
+//    48 sequences x  256 rows:  26.9 / 25.4 / 20.2
+int pick_chunk(long pairs, int cap) {
+    if (cap <= 256 && pairs >= 128) return 256;
     for (int c = kMaxChunk; c > kMinChunk; c >>= 1) {
-        if (pairs * ((bound + c - 1) / c) >= kTargetBlocks) return c;
+        if (pairs * ((cap + c - 1) / c) >= kTargetBlocks) return c;
+    }
+    return cap <= 16 * kMinChunk ? kMinChunk : 2 * kMinChunk;
+}
+
+// An upper bound on the chunks a ring is split into, for the workspace's size:
+// the largest chunk that gives 2048 workgroups, never more than pick_chunk's.
+// (pick_chunk's own counts can fall as the capacity grows, this does not, and
+// one workspace must serve every smaller call.)
+int ws_chunk(long pairs, int bound) {
+    for (int c = kMaxChunk; c > kMinChunk; c >>= 1) {
+        if (pairs * ((bound + c - 1) / c) >= 2048) return c;
     }
     return kMinChunk;
 }
 
 int group_max(int D) { return kMaxGD / D < 8 ? kMaxGD / D : 8; }
 
-template <int D, int GM, int QK>
-void launch_gm(const AttnArgs& a, long batch, hipStream_t st) {
+template <int D, int GM, int QK, int W>
+void launch_w(const AttnArgs& a, long batch, hipStream_t st) {
     if constexpr (GM <= 4) {   // the whole ring's scores within 32 KB of LDS
         if (a.whole_ring) {
             AttnArgs w = a;
             w.nsplit = 1;
             w.chunk = w.whole = a.cap;
-            hipLaunchKernelGGL((gqa_decode_kernel<D, GM, true, QK, kWholeRingMax>), dim3(a.nkv, batch, 1),
-                               dim3(kAttnThreads), 0, st, w);
+            hipLaunchKernelGGL((gqa_decode_kernel<D, GM, true, QK, kWholeRingMax, W>), dim3(a.nkv, batch, 1),
+                               dim3(kWave * W), 0, st, w);
             return;
         }
     }
     const dim3 grid(a.nkv, batch, a.nsplit);
     if (a.nsplit == 1) {
-        hipLaunchKernelGGL((gqa_decode_kernel<D, GM, true, QK>), grid, dim3(kAttnThreads), 0, st, a);
+        hipLaunchKernelGGL((gqa_decode_kernel<D, GM, true, QK, kMaxChunk, W>), grid, dim3(kWave * W), 0, st, a);
     } else {
-        hipLaunchKernelGGL((gqa_decode_kernel<D, GM, false, QK>), grid, dim3(kAttnThreads), 0, st, a);
+        hipLaunchKernelGGL((gqa_decode_kernel<D, GM, false, QK, kMaxChunk, W>), grid, dim3(kWave * W), 0, st, a);
     }
+}
+
+template <int D, int GM, int QK>
+void launch_gm(const AttnArgs& a, long batch, hipStream_t st) {
+    if (a.waves == 8) launch_w<D, GM, QK, 8>(a, batch, st);
+    else launch_w<D, GM, QK, 4>(a, batch, st);
 }
 
 // One launch per slice of at most group_max(D) q heads of each kv head.  A
@@ -608,7 +666,7 @@ size_t ctr_offset(size_t ws_bytes) { return (ws_bytes - ws_bytes / 64) & ~(size_
 size_t ctr_slots(size_t ws_bytes) { return (ws_bytes - ctr_offset(ws_bytes)) / sizeof(unsigned); }
 
 // A size that serves every call with at most `batch` sequences and a ring
-// bound of at most `cap`.  The chunk follows the batch (pick_chunk), so a
+// bound of at most `cap`.  The chunk follows the batch (ws_chunk), so a
 // smaller batch can need more partials than the largest one: the maximum is
 // taken over the batches up to `batch`.  Past the batch at which the chunk
 // reaches its maximum the partials only grow with the batch, so the loop
@@ -616,14 +674,14 @@ size_t ctr_slots(size_t ws_bytes) { return (ws_bytes - ctr_offset(ws_bytes)) / s
 size_t ws_bytes_for(long batch, int nh, int nkv, int D, int cap) {
     size_t P = 0;
     auto count = [&](long b) {
-        const int chunk = pick_chunk(b * nkv, cap);
+        const int chunk = ws_chunk(b * nkv, cap);
         const long nsplit = (cap + chunk - 1) / chunk;
         if (nsplit > 1) {
             const size_t pb = partial_bytes(b, nh, (int)nsplit, D);
             P = pb > P ? pb : P;
         }
     };
-    for (long b = 1; b < batch && pick_chunk(b * nkv, cap) < kMaxChunk; b++) count(b);
+    for (long b = 1; b < batch && ws_chunk(b * nkv, cap) < kMaxChunk; b++) count(b);
     count(batch);
     if (P == 0) return 0;
     const size_t pairs = (size_t)batch * nkv;
@@ -655,6 +713,12 @@ int check_common(const void* out, const void* q, const void* kc, const void* vc,
 // anything is launched.
 int plan(AttnArgs& a, long batch, int D, int bound, void* ws, size_t ws_bytes) {
     a.groups = a.nh / a.nkv;
+    // Eight waves take a chunk in half the rounds of loads of four (64
+    // sequences of ragged lengths up to 2048 rows 109 us against 128, though
+    // all 2048 long 167 against 164; 1 x 512 rows 7.8 against 8.4); four where
+    // every ring is a round or two and the pairs fill the chip anyway (64
+    // sequences x 128 rows: 13.8 against 14.3).
+    a.waves = a.cap <= 128 && batch * a.nkv >= 256 ? 4 : 8;
     a.scale = 1.0f / sqrtf((float)D);   // core/cpu_ops.cpp:183
     a.chunk = pick_chunk(batch * a.nkv, a.cap);  // from the capacity, so the workspace size holds for any bound
     a.nsplit = (bound + a.chunk - 1) / a.chunk;

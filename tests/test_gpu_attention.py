@@ -6,7 +6,7 @@ itself can cancel to ~0); the ring append is bit-exact."""
 import numpy as np
 import pytest
 
-from helpers import assert_bitexact, attention_fp64, dev, host
+from helpers import assert_bitexact, attention_fp64, bf16, dev, host
 
 pytestmark = pytest.mark.gpu
 ATTN_TOL = 1e-5
@@ -334,3 +334,63 @@ def test_workspace_size_covers_smaller_batches(hip):
     caches = torch.zeros(3, cap, nk * D, device="cuda")
     hip.gqa_attention(out, q, caches, caches, z, z, nq, nk, D, ws)
     assert not host(out).any()
+
+
+# Ring lengths around a workgroup's rounds of loads (four waves up to 32 rows,
+# then eight with 64 rows a batch and 128 a double batch), around chunks of 64,
+# 128, 256 and 512 rows and the 128 rows that one workgroup does alone; few
+# pairs (chunks of 64; of 128 past 16 chunks), enough for larger ones, rings of
+# up to 256 rows unsplit, and 256 pairs of short rings (four waves throughout).
+@pytest.mark.parametrize("B,nq,nk,cap,lens", [
+    (12, 16, 8, 512, [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 512]),
+    (2, 8, 4, 1100, [1100, 897]), (8, 8, 8, 1024, [1024, 129, 255, 256, 257, 384, 385, 640]),
+    (16, 20, 4, 256, [256, 1, 33, 65, 128, 129, 192, 193] * 2), (40, 8, 8, 1000, [1000, 512, 513, 300] * 10),
+    (64, 4, 4, 128, [128, 1, 31, 32, 33, 64, 65, 127] * 8)])
+def test_chunk_and_batch_edges(hip, orc, rng, B, nq, nk, cap, lens):
+    """The fused q/k norm + RoPE + append + attention against the separate
+    calls bit for bit (outputs, caches), and those against the oracle, with
+    the newest row anywhere in a chunk; the workspace's counters end at zero."""
+    import torch
+
+    D, lens = 128, np.array(lens, np.int32)
+    starts = rng.integers(0, cap, B).astype(np.int32)
+    starts[0] = cap - 1
+    qkv = rng.standard_normal((B, (nq + 2 * nk) * D)).astype(np.float32)
+    pos = rng.integers(0, 3000, B).astype(np.int32)
+    w = [dev(bf16(1 + 0.1 * rng.standard_normal(D)).view(np.int16)).view(torch.bfloat16) for _ in range(2)]
+    c_tab, s_tab = (dev(t) for t in orc.rope_table(2048, D, 1e6))
+    kc0 = rng.standard_normal((B, cap, nk * D)).astype(np.float32)
+    vc0 = rng.standard_normal((B, cap, nk * D)).astype(np.float32)
+    before = np.maximum(lens - 1, 0)   # the append brings each ring to lens rows (an empty one to one)
+    lens = before + 1
+    ws = torch.zeros(max(hip.gqa_workspace_size(B, nq, nk, D, cap), 16), dtype=torch.uint8, device="cuda")
+    res = []
+    for fused in (False, True):
+        a, kc, vc, rs, rl = dev(qkv), dev(kc0), dev(vc0), dev(starts), dev(before)
+        q, k, v = a[:, :nq * D], a[:, nq * D:(nq + nk) * D], a[:, (nq + nk) * D:]
+        out = torch.full((B, nq * D), float("nan"), device="cuda")
+        if fused:
+            hip.gqa_attention_qk(out, q, k, v, *w, dev(pos), c_tab, s_tab, kc, vc, rs, rl, nq, nk, ws, 1e6, 1e-6, advance=True)
+        else:
+            hip.qknorm_rope_append(q, k, v, *w, dev(pos), c_tab, s_tab, kc, vc, rs, rl, 1e6, 1e-6, nq=nq, nk=nk)
+            qn = host(q.contiguous())
+            hip.gqa_attention(out, q, kc, vc, rs, rl, nq, nk, D, ws)
+        res.append([host(t) for t in (out, kc, vc, rs, rl)])
+    for name, x, y in zip(("out", "k", "v", "start", "len"), *res):
+        assert_bitexact(y, x, f"fused vs separate: {name}")
+    assert np.array_equal(res[0][4], lens)
+    for b in range(B):
+        check(res[0][0][b].reshape(nq, D), qn[b], res[0][1][b], res[0][2][b], nq, nk, D, int(res[0][3][b]), int(lens[b]), orc)
+    n = ws.numel()
+    assert not host(ws)[_ctr_region(n):].any()
+
+
+@pytest.mark.parametrize("D,nq,nk", [(64, 8, 2), (256, 8, 2), (256, 4, 4), (64, 16, 2)])
+def test_slot_sums_other_widths(hip, orc, rng, D, nq, nk):
+    """The sums over a wave's position slots at 8 and 32 lanes per position,
+    with rings that leave some slots and waves without a row."""
+    B, cap = 6, 400
+    starts, lens = rng.integers(0, cap, B), [1, 3, 17, 65, 200, 400]
+    got, q, kc, vc = batched(hip, B, nq, nk, D, cap, starts, lens, rng)
+    for b in range(B):
+        check(got[b], q[b], kc[b], vc[b], nq, nk, D, int(starts[b]), lens[b], orc)
