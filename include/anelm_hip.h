@@ -545,7 +545,7 @@ long anelm_write_ane_blobs(const char* safetensors_path, const char* output_dir,
  * row-major fp16, fp32 accumulation, one rounding to nearest.  Any shape
  * and alignment; in_dim a multiple of 32 with 16-byte aligned rows takes the
  * MFMA kernels (past 16 rows against a long W, x staged in LDS so each weight
- * row is read once for every row of x). */
+ * row is read once for every row of x; for a prompt, block tiles). */
 int anelm_linear_f16(uint16_t* y16, const uint16_t* x16, const uint16_t* w16, long batch, int out_dim, int in_dim,
                      long ld_x, long ld_y, void* stream);
 
