@@ -42,7 +42,12 @@ __device__ __forceinline__ uint32_t f16_bits_rne(float v) {
 // RMSNorm and 7 for add + RMSNorm at 8192 rows of 4096.)
 // TILE (with O16, dim a multiple of 32): the fp16 output in the tiled layout
 // of anelm_proj_tile_f16 (rows of 16, steps of 32 columns, each 16 x 32 block
-// one contiguous 1 KB piece), the input layout of the tiled projection.
+// one contiguous 1 KB piece), the input layout of the tiled projection.  A row
+// writes 16 bytes of each 128-byte line there and seven neighbours the rest,
+// so rows in launch order, dealt to the 8 XCDs in turn, sent every line to
+// memory in eight parts.  In a grid of whole 64s, workgroup i takes row
+// 8 * (i % 8) + (i / 8) % 8 of its 64, so each XCD's L2 gathers whole lines:
+// 2048 x 4096 21.5 -> 15.2 us, 500 x 2560 5.2 -> 4.0, 48 x 1024 2.06 -> 2.00.
 template <int NV, int DT, bool ADD, bool O16 = false, bool FULL = false, bool TILE = false>
 __global__ __launch_bounds__(1024) void rmsnorm_row_kernel(void* out, float* x, const float* y,
                                                            const void* w, long rows, int dim,
@@ -50,7 +55,11 @@ __global__ __launch_bounds__(1024) void rmsnorm_row_kernel(void* out, float* x, 
                                                            float eps) {
     __shared__ float part[16];
     const int tid = threadIdx.x, nthr = blockDim.x;
-    const long row = blockIdx.x;
+    long row = blockIdx.x;
+    if (TILE && (gridDim.x & 63) == 0) {
+        row = (row & ~63L) | ((row & 7) << 3) | ((row >> 3) & 7);
+        if (row >= rows) return;
+    }
     float* xr = x + row * ld_x;
     int col[NV];
     bool live[NV];
@@ -172,7 +181,9 @@ static int launch_rmsnorm_dt(void* out, float* x, const float* y, const void* w,
     if (vec && nvec <= 1024 * 4) {
         int nv, threads;
         rms_row_geometry(rows, nvec, nv, threads);
-        const dim3 grd((unsigned)rows);
+        // Whole 64s for the tiled rows' order: not for a single tile, nor past
+        // 2^24 rows, where rounding up could pass the grid's limit.
+        const dim3 grd((unsigned)(TILE && rows > 16 && rows <= (1L << 24) ? (rows + 63) / 64 * 64 : rows));
         const bool full = nvec == nv * threads;
 #define ANELM_RMS_ROW(NV_, FULL_) \
     rmsnorm_row_kernel<NV_, DT, ADD, O16, FULL_, TILE><<<grd, threads, 0, st>>>(out, x, y, w, rows, dim, ld_x, ld_y, ld_out, eps)

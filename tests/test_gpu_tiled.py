@@ -28,7 +28,7 @@ def tiled_buf(rows, cols):
     return torch.full(((rows + 15) // 16 * 16 * cols,), -1, dtype=torch.int16, device="cuda")
 
 
-@pytest.mark.parametrize("rows,dim", [(64, 1024), (17, 1024), (33, 4096), (5, 96), (100, 2048)])
+@pytest.mark.parametrize("rows,dim", [(64, 1024), (17, 1024), (33, 4096), (5, 96), (100, 2048), (9, 96), (65, 1024), (130, 4096)])
 def test_rmsnorm_f16_tiled(hip, rng, rows, dim):
     import torch
 
