@@ -47,7 +47,7 @@ __device__ __forceinline__ uint32_t f16_bits_rne(float v) {
 // so rows in launch order, dealt to the 8 XCDs in turn, sent every line to
 // memory in eight parts.  In a grid of whole 64s, workgroup i takes row
 // 8 * (i % 8) + (i / 8) % 8 of its 64, so each XCD's L2 gathers whole lines:
-// 2048 x 4096 21.5 -> 15.2 us, 500 x 2560 5.2 -> 4.0, 48 x 1024 2.06 -> 2.00.
+// 2048 x 4096 21.5 -> 15.2 us, 500 x 2560 5.2 -> 4.0, 300 x 1024 2.5 -> 2.2.
 template <int NV, int DT, bool ADD, bool O16 = false, bool FULL = false, bool TILE = false>
 __global__ __launch_bounds__(1024) void rmsnorm_row_kernel(void* out, float* x, const float* y,
                                                            const void* w, long rows, int dim,
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_row_kernel(void* out, float* x, 
     __shared__ float part[16];
     const int tid = threadIdx.x, nthr = blockDim.x;
     long row = blockIdx.x;
-    if (TILE && (gridDim.x & 63) == 0) {
+    if (TILE && rows >= 128 && (gridDim.x & 63) == 0) {
         row = (row & ~63L) | ((row & 7) << 3) | ((row >> 3) & 7);
         if (row >= rows) return;
     }
@@ -181,9 +181,10 @@ static int launch_rmsnorm_dt(void* out, float* x, const float* y, const void* w,
     if (vec && nvec <= 1024 * 4) {
         int nv, threads;
         rms_row_geometry(rows, nvec, nv, threads);
-        // Whole 64s for the tiled rows' order: not for a single tile, nor past
-        // 2^24 rows, where rounding up could pass the grid's limit.
-        const dim3 grd((unsigned)(TILE && rows > 16 && rows <= (1L << 24) ? (rows + 63) / 64 * 64 : rows));
+        // Whole 64s for the tiled rows' order: not below 128 rows (a decode step
+        // of 64 sequences took 1.107 ms without it, 1.109 with), nor past 2^24
+        // rows, where rounding up could pass the grid's limit.
+        const dim3 grd((unsigned)(TILE && rows >= 128 && rows <= (1L << 24) ? (rows + 63) / 64 * 64 : rows));
         const bool full = nvec == nv * threads;
 #define ANELM_RMS_ROW(NV_, FULL_) \
     rmsnorm_row_kernel<NV_, DT, ADD, O16, FULL_, TILE><<<grd, threads, 0, st>>>(out, x, y, w, rows, dim, ld_x, ld_y, ld_out, eps)
