@@ -184,6 +184,16 @@ def _stream(stream):
     return _raw_stream()
 
 
+def _forget_raw_stream():
+    global _raw_stream
+    _raw_stream = None
+
+
+# HIP does not survive a fork.  torch.cuda.current_stream() raises in a forked
+# child, the raw handle does not: the child asks torch again.
+os.register_at_fork(after_in_child=_forget_raw_stream)
+
+
 _dtype_codes = {}
 
 

@@ -315,3 +315,30 @@ def test_rmsnorm_geometry_at_the_workload_shapes():
     assert anelm.rmsnorm_geometry(4, 1022) == (0, 256)        # not a multiple of 4: the any-shape kernel
     with pytest.raises(anelm.AnelmError):
         anelm.rmsnorm_geometry(0, 1024)
+
+
+def test_forked_child_asks_torch_for_its_stream(monkeypatch):
+    """A process that has used the GPU keeps a getter of the raw stream handle;
+    in a forked child, where HIP is unusable, torch.cuda.current_stream()
+    raises, and so must every call (stand-ins for both: no GPU here)."""
+    import torch
+
+    import anelm
+
+    def refuse():
+        raise RuntimeError("Cannot re-initialize CUDA in forked subprocess")
+
+    monkeypatch.setattr(anelm, "_raw_stream", lambda: 7)
+    monkeypatch.setattr(torch.cuda, "current_stream", refuse)
+    assert anelm._stream(None) == 7
+    pid = os.fork()
+    if pid == 0:
+        code = 1
+        try:
+            anelm._stream(None)
+        except RuntimeError:
+            code = 0
+        finally:
+            os._exit(code)
+    assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0, "the child used the parent's stream"
+    assert anelm._stream(None) == 7
