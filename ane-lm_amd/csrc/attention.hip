@@ -26,12 +26,14 @@
 // With many (sequence, kv head) pairs and rings of at most 2048 rows, one
 // workgroup per pair takes the whole ring instead (the same phases over up
 // to 2048 positions), and nothing is merged.
+#include <algorithm>
+
 #include "anelm_common.hpp"
+#include "attention_plan.hpp"
 
 namespace anelm {
 namespace {
 
-constexpr int kMaxChunk = 512;        // ring positions per workgroup of a split launch
 // Whole-ring launches: with at least kWholeRingPairs (sequence, kv head)
 // pairs (two per CU) and rings of at most kWholeRingMax rows, one workgroup
 // per pair attends over the whole ring and writes the output itself: no
@@ -41,11 +43,8 @@ constexpr int kMaxChunk = 512;        // ring positions per workgroup of a split
 // pairs per CU some CUs would run two rings and others one.
 constexpr int kWholeRingMax = 2048;
 constexpr long kWholeRingPairs = 512;
-constexpr int kMinChunk = 64;
 constexpr int kMaxGD = 1024;          // group heads x head_dim per workgroup
-constexpr long kTargetBlocks = 384;   // workgroups of a split launch (see pick_chunk)
 constexpr int kMaxSplit = 4096;       // chunks per sequence (capacity <= 4096*32)
-constexpr int kWholeRows = 128;       // rings up to this long (or one chunk) are done by one workgroup
 static_assert(kWholeRows <= kMaxChunk, "a whole ring's scores fit the LDS rows");
 
 struct AttnArgs {
@@ -64,8 +63,8 @@ struct AttnArgs {
     long out_ld;                // between sequences; heads are head_dim apart
     int cap;
     long seq_stride;            // between sequences' caches
-    int chunk, nsplit;
-    int whole;                  // split launches: rings of at most this many rows are done by chunk 0 alone
+    int nsplit;                 // chunks launched (and partials kept) per sequence
+    int pairs;                  // (sequence, kv head) pairs, at most kMaxPairs: with a ring's length, its chunk
     int g0, gcount;             // q heads g0 .. g0+gcount-1 of every group
     float scale;
     float* ws;                  // [batch*nh][nsplit][head_dim + 2] partials
@@ -170,7 +169,7 @@ template <int D>
 __device__ void merge_head(const AttnArgs& a, long b, int h, int lane, int live) {
     // Chunks whose partials are in flight at once: 32 held 64 more registers
     // through the whole kernel (3 waves per SIMD instead of 5) for a merge that
-    // pick_chunk keeps to a few batches (16 x 1024 ragged rows 26.9 -> 24.6 us).
+    // ring_chunk keeps to a few batches (16 x 1024 ragged rows 26.9 -> 24.6 us).
     constexpr int kBatch = 8;
     const int ns = a.nsplit;
     const float* p = a.ws + (b * a.nh + h) * ns * (long)(D + 2);
@@ -289,15 +288,16 @@ __global__ __launch_bounds__(kWave* W) void gqa_decode_kernel(AttnArgs a) {
     const int qpos = QK >= 0 ? a.pos[b] : 0;   // read beside the ring state
     int start, len;
     ring_state(a, b, start, len);
-    // In a split launch a ring that is short (len <= a.whole, at most one
-    // chunk's worth of LDS) is done by chunk 0 alone, which then writes the
-    // normalised output itself, with no partials and no count.  The ring
-    // lengths live on the device, so this is decided per sequence here.
-    const bool whole = !FINAL && len <= a.whole;
+    // The ring lengths live on the device, so a split launch chooses each
+    // sequence's chunk here.  A ring of one chunk, or of kWholeRows, is done
+    // by chunk 0 alone, which then writes the normalised output itself, with
+    // no partials and no count.
+    const int chunk = FINAL ? MC : ring_chunk(a.pairs, len);
+    const bool whole = !FINAL && len <= max(chunk, kWholeRows);
     if (whole && split > 0) return;
     const bool fin = FINAL || whole;
-    const int t0 = split * a.chunk;
-    const int n = whole ? len : min(t0 + a.chunk, len) - t0;     // positions of this chunk
+    const int t0 = split * chunk;
+    const int n = whole ? len : min(t0 + chunk, len) - t0;     // positions of this chunk
     if (!fin && n <= 0) return;   // past the ring: neither partials nor a count
     // a chunk that four waves take in one batch is left to them: the others'
     // share of the set-up and of the barriers costs more than they would save
@@ -521,7 +521,7 @@ __global__ __launch_bounds__(kWave* W) void gqa_decode_kernel(AttnArgs a) {
         // A bounded launch can hold fewer chunks than a ring longer than its
         // bound needs: then the nsplit launched chunks are the live ones.
         __shared__ int s_last;
-        const int live = min((len + a.chunk - 1) / a.chunk, a.nsplit);
+        const int live = min(ring_chunks(a.pairs, len), a.nsplit);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         if (tid == 0) {
@@ -573,41 +573,6 @@ __global__ __launch_bounds__(256) void kv_ring_advance_kernel(int32_t* rs, int32
     ring_advance(rs + r, rl + r, cap);
 }
 
-// Positions per workgroup for rings of `cap` positions and `pairs` (sequence,
-// kv head) pairs.  A split ring costs its last workgroup three more memory
-// round trips (partials stored, counted, read back: 2 us), and merging them
-// takes longer the more there are; a CU pulls a ring in at no more than about
-// 45 GB/s, whatever its waves, so few workgroups are slow too.  The largest
-// chunk that gives kTargetBlocks workgroups; below that 64 positions (128 for
-// rings of more than 16 such chunks); and rings of up to 256 rows are not
-// split at all once half the CUs have one.  us per launch with chunks of
-// 64 / 128 / 256 / 512 (8 waves, 8 kv heads, fused q/k norm):
-//     1 sequence  x  512 rows:   7.8 /  9.3 / 12.4 / 16.7
-//     1 sequence  x 2048 rows:  12.6 / 11.8 / 14.1 / 20.9
-//     8 sequences x 1024 rows:  18.2 / 13.5 / 15.0 / 21.5   (ragged lengths)
-//    16 sequences x 1024 rows:  27.2 / 23.2 / 20.1 / 23.1   (ragged lengths)
-//    48 sequences x 2048 rows: 115   / 93   / 82   / 79     (ragged lengths)
-//    20 sequences x  256 rows:  15.3 / 13.9 / 12.5
-//    48 sequences x  256 rows:  26.9 / 25.4 / 20.2
-int pick_chunk(long pairs, int cap) {
-    if (cap <= 256 && pairs >= 128) return 256;
-    for (int c = kMaxChunk; c > kMinChunk; c >>= 1) {
-        if (pairs * ((cap + c - 1) / c) >= kTargetBlocks) return c;
-    }
-    return cap <= 16 * kMinChunk ? kMinChunk : 2 * kMinChunk;
-}
-
-// An upper bound on the chunks a ring is split into, for the workspace's size:
-// the largest chunk that gives 2048 workgroups, never more than pick_chunk's.
-// (pick_chunk's own counts can fall as the capacity grows, this does not, and
-// one workspace must serve every smaller call.)
-int ws_chunk(long pairs, int bound) {
-    for (int c = kMaxChunk; c > kMinChunk; c >>= 1) {
-        if (pairs * ((bound + c - 1) / c) >= 2048) return c;
-    }
-    return kMinChunk;
-}
-
 int group_max(int D) { return kMaxGD / D < 8 ? kMaxGD / D : 8; }
 
 template <int D, int GM, int QK, int W>
@@ -616,7 +581,6 @@ void launch_w(const AttnArgs& a, long batch, hipStream_t st) {
         if (a.whole_ring) {
             AttnArgs w = a;
             w.nsplit = 1;
-            w.chunk = w.whole = a.cap;
             hipLaunchKernelGGL((gqa_decode_kernel<D, GM, true, QK, kWholeRingMax, W>), dim3(a.nkv, batch, 1),
                                dim3(kWave * W), 0, st, w);
             return;
@@ -638,7 +602,7 @@ void launch_gm(const AttnArgs& a, long batch, hipStream_t st) {
 
 // One launch per slice of at most group_max(D) q heads of each kv head.  A
 // QK launch writes the newest cache row in every slice's launch (the same
-// bits each time) and uses it from registers, so no launch depends on the
+// bits each time) and uses its own copy in LDS, so no launch depends on the
 // order of the others.
 template <int D, int QK = -1>
 void launch_d(AttnArgs a, long batch, hipStream_t st) {
@@ -651,44 +615,6 @@ void launch_d(AttnArgs a, long batch, hipStream_t st) {
         else if (a.gcount <= 4) launch_gm<D, 4, QK>(a, batch, st);
         else launch_gm<D, (kMaxGD / D < 8 ? kMaxGD / D : 8), QK>(a, batch, st);
     }
-}
-
-// Split launches: the partials from the workspace's start, and one counter
-// per (sequence, kv head) in a region whose place depends on the workspace's
-// size alone: its last 64th, from a 256-byte boundary.  Every call given the
-// same workspace and size therefore finds each counter at the same address,
-// left at zero by the calls before, whatever its batch, chunking or ring
-// lengths, and no call's partials reach into the region (checked per call).
-size_t partial_bytes(long batch, int nh, int nsplit, int D) {
-    return ((size_t)batch * nh * nsplit * (D + 2) * sizeof(float) + 255) & ~(size_t)255;
-}
-size_t ctr_offset(size_t ws_bytes) { return (ws_bytes - ws_bytes / 64) & ~(size_t)255; }
-size_t ctr_slots(size_t ws_bytes) { return (ws_bytes - ctr_offset(ws_bytes)) / sizeof(unsigned); }
-
-// A size that serves every call with at most `batch` sequences and a ring
-// bound of at most `cap`.  The chunk follows the batch (ws_chunk), so a
-// smaller batch can need more partials than the largest one: the maximum is
-// taken over the batches up to `batch`.  Past the batch at which the chunk
-// reaches its maximum the partials only grow with the batch, so the loop
-// stops there and `batch` itself is counted last.
-size_t ws_bytes_for(long batch, int nh, int nkv, int D, int cap) {
-    size_t P = 0;
-    auto count = [&](long b) {
-        const int chunk = ws_chunk(b * nkv, cap);
-        const long nsplit = (cap + chunk - 1) / chunk;
-        if (nsplit > 1) {
-            const size_t pb = partial_bytes(b, nh, (int)nsplit, D);
-            P = pb > P ? pb : P;
-        }
-    };
-    for (long b = 1; b < batch && ws_chunk(b * nkv, cap) < kMaxChunk; b++) count(b);
-    count(batch);
-    if (P == 0) return 0;
-    const size_t pairs = (size_t)batch * nkv;
-    size_t S = (((P + 256) * 64 / 63 + 256) + 255) & ~(size_t)255;
-    if (S < 256 * pairs) S = 256 * pairs;
-    while (ctr_offset(S) < P || ctr_slots(S) < pairs) S += 256;
-    return S;
 }
 
 int check_common(const void* out, const void* q, const void* kc, const void* vc, long batch, int nh, int nkv,
@@ -713,23 +639,26 @@ int check_common(const void* out, const void* q, const void* kc, const void* vc,
 // anything is launched.
 int plan(AttnArgs& a, long batch, int D, int bound, void* ws, size_t ws_bytes) {
     a.groups = a.nh / a.nkv;
+    a.scale = 1.0f / sqrtf((float)D);   // core/cpu_ops.cpp:183
+    a.pairs = (int)std::min(batch * a.nkv, (long)kMaxPairs);
+    a.nsplit = batch > 0 ? max_chunks(a.pairs, bound) : 1;
+    auto serves = [&](int nsplit) {
+        return ws && partial_bytes(batch, a.nh, nsplit, D) <= ctr_offset(ws_bytes) &&
+               (size_t)batch * a.nkv <= ctr_slots(ws_bytes);
+    };
+    // rings that one workgroup can do need no workspace: without one, it does them
+    if (bound <= kMaxChunk && !serves(a.nsplit)) a.nsplit = 1;
     // Eight waves take a chunk in half the rounds of loads of four (64
     // sequences of ragged lengths up to 2048 rows 109 us against 128, though
-    // all 2048 long 167 against 164; 1 x 512 rows 7.8 against 8.4); four where
+    // all 2048 long 171.5 against 169.8; 1 x 512 rows 7.8 against 8.4); four where
     // every ring is a round or two and the pairs fill the chip anyway (64
     // sequences x 128 rows: 13.8 against 14.3).
     a.waves = a.cap <= 128 && batch * a.nkv >= 256 ? 4 : 8;
-    a.scale = 1.0f / sqrtf((float)D);   // core/cpu_ops.cpp:183
-    a.chunk = pick_chunk(batch * a.nkv, a.cap);  // from the capacity, so the workspace size holds for any bound
-    a.nsplit = (bound + a.chunk - 1) / a.chunk;
-    if (a.nsplit < 1) a.nsplit = 1;
-    a.whole = a.chunk > kWholeRows ? a.chunk : kWholeRows;   // <= kMaxChunk, the LDS score rows
     if (a.nsplit > 1) {
-        const size_t pb = partial_bytes(batch, a.nh, a.nsplit, D);
-        if (!ws || pb > ctr_offset(ws_bytes) || (size_t)batch * a.nkv > ctr_slots(ws_bytes))
+        if (!serves(a.nsplit))
             return fail(ANELM_ERR_WORKSPACE,
                         "gqa_attention: workspace of %zu bytes too small for %zu bytes of partials and %ld counters",
-                        ws_bytes, pb, batch * a.nkv);
+                        ws_bytes, partial_bytes(batch, a.nh, a.nsplit, D), batch * a.nkv);
         if (!aligned16(ws)) return fail(ANELM_ERR_INVALID, "gqa_attention: workspace not 16-byte aligned");
         a.ctr = reinterpret_cast<unsigned*>(static_cast<char*>(ws) + ctr_offset(ws_bytes));
     }

@@ -314,6 +314,9 @@ int anelm_kv_ring_append(float* k_cache, float* v_cache, int32_t* ring_start, in
  * anelm_gqa_workspace_size(batch, n_heads, n_kv_heads, head_dim, capacity)
  * bytes of device workspace (0 is possible: then workspace may be NULL),
  * zero-filled before its first use (e.g. hipMemset once after allocating).
+ * With less, capacities (or bounds, below) of at most 512 rows are attended by
+ * one workgroup per sequence and kv head, which is slower; longer ones are
+ * ANELM_ERR_WORKSPACE.
  * That size serves every call with at most `batch` sequences and rings of at
  * most `capacity` rows.  The workspace's last 64th holds per-(sequence, kv
  * head) counters of the chunks of a long ring, at addresses that depend only

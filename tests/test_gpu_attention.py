@@ -105,8 +105,8 @@ def test_batched_decode_b64_full_shape(hip, orc, rng):
 
 
 def test_whole_ring_threshold(hip, orc, rng):
-    """Rings short enough for one workgroup (128 rows at this shape: 32-row
-    chunks) are done by chunk 0 alone, longer ones split and merged; lengths
+    """Rings short enough for one workgroup (128 rows: this shape's chunks are
+    of 64 there) are done by chunk 0 alone, longer ones split and merged; lengths
     on both sides of the threshold in one launch, some wrapping."""
     B, nq, nk, D, cap = 6, 16, 8, 128, 2048
     lens = [0, 1, 127, 128, 129, 2048]
@@ -293,9 +293,9 @@ def test_workspace_reuse_across_shapes(hip, orc, rng):
 
 def test_bounded_launch_ring_past_bound(hip, orc, rng):
     """A bounded launch given a ring longer than its bound attends over the
-    launched chunks' positions only: one sequence, 8 kv heads and capacity
-    2048 give 64-position chunks, so a bound of 200 launches 4 chunks and a
-    700-row ring is attended over its first 256 positions.  The counters are
+    launched chunks' positions only: one sequence and 8 kv heads give
+    64-position chunks up to 1024 rows, so a bound of 200 launches 4 chunks and
+    a 700-row ring is attended over its first 256 positions.  The counters are
     left at zero: a full call on the same workspace afterwards is right."""
     import torch
 
@@ -337,15 +337,23 @@ def test_workspace_size_covers_smaller_batches(hip):
 
 
 # Ring lengths around a workgroup's rounds of loads (four waves up to 32 rows,
-# then eight with 64 rows a batch and 128 a double batch), around chunks of 64,
-# 128, 256 and 512 rows and the 128 rows that one workgroup does alone; few
-# pairs (chunks of 64; of 128 past 16 chunks), enough for larger ones, rings of
-# up to 256 rows unsplit, and 256 pairs of short rings (four waves throughout).
+# then eight with 64 rows a batch and 128 a double batch), the 128 rows that one
+# workgroup does alone, and the lines of the chunk rule: 64 | 128 rows a chunk
+# at 256 | 257 rows with 64 pairs, 341 | 342 with 48, 1024 | 1025 with 8; 128 |
+# 256 at 1562 | 1563 with 48, 585 | 586 with 128; 256 | 512 at 687 | 688 with
+# 320; rings of up to 256 rows unsplit past 128 pairs (a capacity of 256: one
+# launch without a split), of up to 512 from 256 pairs; 256 pairs of short rings
+# (four waves throughout); a long capacity with a short ring; groups of 8 q
+# heads with eight waves and with four.
 @pytest.mark.parametrize("B,nq,nk,cap,lens", [
     (12, 16, 8, 512, [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 512]),
-    (2, 8, 4, 1100, [1100, 897]), (8, 8, 8, 1024, [1024, 129, 255, 256, 257, 384, 385, 640]),
-    (16, 20, 4, 256, [256, 1, 33, 65, 128, 129, 192, 193] * 2), (40, 8, 8, 1000, [1000, 512, 513, 300] * 10),
-    (64, 4, 4, 128, [128, 1, 31, 32, 33, 64, 65, 127] * 8)])
+    (3, 8, 4, 1100, [1100, 897, 340]), (8, 8, 8, 1024, [1024, 129, 255, 256, 257, 384, 385, 640]),
+    (1, 8, 8, 8192, [500]), (2, 8, 4, 1100, [1024, 1025]),
+    (6, 16, 8, 2048, [341, 342, 1562, 1563, 2048, 256]), (16, 20, 4, 256, [256, 1, 33, 65, 128, 129, 192, 193] * 2),
+    (32, 8, 4, 600, [128, 129, 256, 257, 512, 513, 585, 586] * 4), (33, 8, 4, 256, [256, 129, 128] * 11),
+    (33, 8, 4, 300, [255, 256, 257] * 11), (40, 8, 8, 1000, [1000, 512, 513, 687, 688] * 8),
+    (64, 4, 4, 128, [128, 1, 31, 32, 33, 64, 65, 127] * 8),
+    (3, 16, 2, 400, [400, 129, 64]), (20, 16, 2, 1100, [1100, 614, 128, 129, 900] * 4)])
 def test_chunk_and_batch_edges(hip, orc, rng, B, nq, nk, cap, lens):
     """The fused q/k norm + RoPE + append + attention against the separate
     calls bit for bit (outputs, caches), and those against the oracle, with
@@ -383,6 +391,49 @@ def test_chunk_and_batch_edges(hip, orc, rng, B, nq, nk, cap, lens):
         check(res[0][0][b].reshape(nq, D), qn[b], res[0][1][b], res[0][2][b], nq, nk, D, int(res[0][3][b]), int(lens[b]), orc)
     n = ws.numel()
     assert not host(ws)[_ctr_region(n):].any()
+
+
+@pytest.mark.parametrize("B,nk,cap", [(1, 8, 1024), (2, 8, 1024), (1, 1, 700)])
+def test_workspace_filled(hip, orc, rng, B, nk, cap):
+    """Rings whose chunks fill the workspace's partials to the last one (64
+    rows each, what the size counts): right, and nothing past the end."""
+    import torch
+
+    nq, D = 2 * nk, 128
+    n = hip.gqa_workspace_size(B, nq, nk, D, cap)
+    assert n >= B * nq * -(-cap // 64) * (D + 2) * 4
+    buf = torch.zeros(n + 4096, dtype=torch.uint8, device="cuda")
+    buf[n:] = 0xA5
+    q = rng.standard_normal((B, nq * D)).astype(np.float32)
+    kc, vc = (rng.standard_normal((B, cap, nk * D)).astype(np.float32) for _ in range(2))
+    starts = rng.integers(0, cap, B).astype(np.int32)
+    out = torch.full((B, nq * D), float("nan"), device="cuda")
+    hip.gqa_attention(out, dev(q), dev(kc), dev(vc), dev(starts), dev(np.full(B, cap, np.int32)), nq, nk, D, buf[:n])
+    for b in range(B):
+        check(host(out)[b].reshape(nq, D), q[b], kc[b], vc[b], nq, nk, D, int(starts[b]), cap, orc)
+    assert bool((buf[n:] == 0xA5).all()) and not host(buf)[_ctr_region(n):n].any()
+
+
+def test_without_workspace(hip, orc, rng):
+    """Rings of at most 512 rows are served without a workspace, by one
+    workgroup each; past that, too small a one is an error."""
+    import torch
+
+    B, nq, nk, D, none = 2, 8, 4, 128, torch.zeros(16, dtype=torch.uint8, device="cuda")
+    for cap in (300, 512, 513):
+        q = rng.standard_normal((B, nq * D)).astype(np.float32)
+        kc, vc = (rng.standard_normal((B, cap, nk * D)).astype(np.float32) for _ in range(2))
+        starts, lens = np.array([7, 250], np.int32), np.array([cap, 200], np.int32)
+        out = torch.full((B, nq * D), float("nan"), device="cuda")
+        args = (out, dev(q), dev(kc), dev(vc), dev(starts), dev(lens), nq, nk, D)
+        if cap > 512:
+            with pytest.raises(hip.AnelmError) as e:
+                hip.gqa_attention(*args, none)
+            assert e.value.code == hip.ERR_WORKSPACE
+            continue
+        hip.gqa_attention(*args, none)
+        for b in range(B):
+            check(host(out)[b].reshape(nq, D), q[b], kc[b], vc[b], nq, nk, D, int(starts[b]), int(lens[b]), orc)
 
 
 @pytest.mark.parametrize("D,nq,nk", [(64, 8, 2), (256, 8, 2), (256, 4, 4), (64, 16, 2)])
