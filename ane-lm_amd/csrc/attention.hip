@@ -652,8 +652,13 @@ int plan(AttnArgs& a, long batch, int D, int bound, void* ws, size_t ws_bytes) {
     // sequences of ragged lengths up to 2048 rows 109 us against 128, though
     // all 2048 long 171.5 against 169.8; 1 x 512 rows 7.8 against 8.4); four where
     // every ring is a round or two and the pairs fill the chip anyway (64
-    // sequences x 128 rows: 13.8 against 14.3).
-    a.waves = a.cap <= 128 && batch * a.nkv >= 256 ? 4 : 8;
+    // sequences x 128 rows: 13.8 against 14.3).  With more than four q heads
+    // (158 VGPRs, three waves per SIMD) a CU holds one workgroup of eight waves
+    // but three of four, so four where there are more workgroups than CUs (64
+    // q heads: 32 x 2048 ragged rows 63 us against 82, 3 x 2048 rows 21.6
+    // against 24.8; but 32 x 512 44 against 30, 1 x 2048 19.4 against 14.5).
+    const bool wide = std::min(a.groups, group_max(D)) > 4 && batch * a.nkv * a.nsplit > 256;
+    a.waves = wide || (a.cap <= 128 && batch * a.nkv >= 256) ? 4 : 8;
     if (a.nsplit > 1) {
         if (!serves(a.nsplit))
             return fail(ANELM_ERR_WORKSPACE,
