@@ -635,8 +635,11 @@ int anelm_proj_f16_x16_tiled(void* y, const uint16_t* x16, const uint16_t* w_til
  * SwiGLU result written in the tiled layout (batch rows, out_dim columns, a
  * multiple of 32; ld_y unused), the input of the next anelm_proj_f16_tt.
  * The MFMA kernels of anelm_proj_f16_x16_fused on the same operands: outputs
- * bit-identical to it past 16 rows.  x_t and W 16-byte aligned, in_dim a
- * multiple of 32.  No counterpart in the reference. */
+ * bit-identical to it past 16 rows, except for the stores (ANELM_PROJ_STORE,
+ * ANELM_PROJ_STORE_F16) of 8192 or more outputs with in_dim a multiple of 256
+ * up to 4096, which take a kernel of their own where x is in rows: the same
+ * products, their fp32 sums in another order.  x_t and W 16-byte aligned,
+ * in_dim a multiple of 32.  No counterpart in the reference. */
 #define ANELM_PROJ_SWIGLU_F16_TILED 5
 int anelm_proj_f16_tt(void* y, const uint16_t* x_t, const uint16_t* w_t, long batch, int out_dim, int in_dim,
                       long ld_y, int epilogue, void* stream);

@@ -207,3 +207,41 @@ def test_many_rows(hip, orc, rng, B, out_dim, in_dim):
             assert_bitexact(untile(host(ht), B, n), h16, "tiled fp16 SwiGLU")
             pad = np.asarray(host(ht)).reshape((B + 15) // 16, n // 32, 4, 16, 8)[-1, :, :, (B - 1) % 16 + 1:]
             assert np.all(pad.astype(np.uint16) == 0xFFFF), "rows past the batch are left as they are"
+
+
+# Stores of 8192 or more outputs, all of x in LDS: 64, 32 and 16 rows a
+# workgroup, with rows and outputs that are only partly there.
+@pytest.mark.parametrize("B,out_dim,in_dim", [(17, 8192, 256), (64, 8200, 1024), (30, 8208, 2048), (20, 8196, 4096)])
+def test_stores_through_lds(hip, orc, rng, B, out_dim, in_dim):
+    """Every layout with x in rows gives the same bits here too, in fp32 and
+    fp16; x tiled takes the kernels that split the inputs over waves, whose sums
+    run in another order: its fp16 stores are its fp32 ones, each checked."""
+    import torch
+    from test_gpu_qwen3 import check_projection
+
+    x = (2 * rng.standard_normal((B, in_dim))).astype(np.float32)
+    x16 = orc.f32_to_f16_rne(x).reshape(B, in_dim)
+    w = (0.03 * rng.standard_normal((out_dim, in_dim))).astype(np.float16).view(np.uint16)
+    xr, dw = dev(x16.view(np.int16)), dev(w.view(np.int16))
+    xt, wt = tiled_buf(B, in_dim), tiled_buf(out_dim, in_dim)
+    hip.proj_tile_f16(xt, xr)
+    # the rows past the batch are padding, whatever they hold
+    pad = xt.view((B + 15) // 16, in_dim // 32, 4, 16, 8)[-1, :, :, (B - 1) % 16 + 1:]
+    pad.fill_(0x7E00)
+    hip.proj_tile_f16(wt, dw)
+    out = lambda dt: torch.full((B, out_dim), -1, dtype=dt, device="cuda")  # noqa: E731
+    y = [out(torch.float32) for _ in range(4)]
+    hip.proj_f16_x16_fused(y[0], xr, dw)
+    hip.proj_f16_x16(y[1], xr, dw)
+    hip.proj_f16_x16_tiled(y[2], xr, wt, out_dim)
+    hip.proj_f16_tt(y[3], xt, wt, B, out_dim, in_dim, epilogue=hip.PROJ_STORE)
+    check_projection(orc, x, w, host(y[0]).astype(np.float64))
+    check_projection(orc, x, w, host(y[3]).astype(np.float64))
+    for i in (1, 2):
+        assert_bitexact(host(y[i]), host(y[0]), f"layout {i}")
+    h = [out(torch.int16) for _ in range(3)]
+    hip.linear_f16(h[0], xr, dw)
+    hip.proj_f16_x16_tiled(h[1], xr, wt, out_dim, epilogue=hip.PROJ_STORE_F16)
+    hip.proj_f16_tt(h[2], xt, wt, B, out_dim, in_dim, epilogue=hip.PROJ_STORE_F16)
+    for i, of in enumerate((y[0], y[0], y[3])):
+        assert_bitexact(host(h[i]), orc.f32_to_f16_rne(host(of)).reshape(B, out_dim).view(np.int16), f"fp16 store {i}")
