@@ -67,3 +67,45 @@ def test_few_rows(hip, orc, rng, B, out_dim, in_dim):
         if norm is None:
             hip.proj_f16_x16_fused(h, xh, dw[:2 * n], epilogue=hip.PROJ_SWIGLU)
             assert_bitexact(orc.f32_to_f16_rne(host(h)).reshape(B, n), host(h16), "SwiGLU of fp16 rows vs fp32 rows")
+
+
+# 7 and 16 rows: the kernel above; 40: proj_mfma_kernel; 100: block tiles.
+@pytest.mark.parametrize("B", [7, 16, 40, 100])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_rows_do_not_mix(hip, rng, B, bad):
+    """A NaN or an infinity in a row of x, or of W, reaches that row's outputs
+    (that column's) and no others: these keep their bits."""
+    import torch
+
+    out_dim, in_dim = 4112, 160
+    x = rng.standard_normal((B, in_dim)).astype(np.float32)
+    w = (0.03 * rng.standard_normal((out_dim, in_dim))).astype(np.float16)
+    xb, wb = x.copy(), w.copy()
+    rows, cols = [2, B - 1], [0, 2055, 4111]
+    xb[rows, [5, in_dim - 1]] = bad
+    wb[cols, [0, 33, in_dim - 1]] = bad
+    gamma = dev(bf16(np.ones(in_dim, np.float32)).view(np.int16))
+    tiled = lambda a: torch.zeros((a.shape[0] + 15) // 16 * 16 * a.shape[1], dtype=torch.int16, device="cuda")  # noqa: E731
+
+    def calls(x, w):
+        xf, dw = dev(x), dev(w.view(np.int16))
+        xh = xf.half().view(torch.int16)
+        wt, xt = tiled(w), tiled(x)
+        hip.proj_tile_f16(wt, dw)
+        hip.proj_tile_f16(xt, xh)
+        ys = [torch.zeros(B, out_dim, device="cuda") for _ in range(5)]
+        hip.proj_f16_fused(ys[0], xf, dw)
+        hip.proj_f16_fused(ys[1], xf, dw, norm=gamma, eps=1e-6)
+        hip.proj_f16_x16_fused(ys[2], xh, dw)
+        hip.proj_f16_x16_tiled(ys[3], xh, wt, out_dim)
+        hip.proj_f16_tt(ys[4], xt, wt, B, out_dim, in_dim, epilogue=hip.PROJ_STORE)
+        return [host(y) for y in ys]
+
+    clean = calls(x, w)
+    for i, (y, of_x, of_w) in enumerate(zip(clean, calls(xb, w), calls(x, wb))):
+        keep = np.setdiff1d(np.arange(B), rows)
+        assert_bitexact(of_x[keep], y[keep], f"call {i}: other rows")
+        assert not np.isfinite(of_x[rows]).any(), f"call {i}: rows of the {bad}"
+        keep = np.setdiff1d(np.arange(out_dim), cols)
+        assert_bitexact(of_w[:, keep], y[:, keep], f"call {i}: other columns")
+        assert not np.isfinite(of_w[:, cols]).any(), f"call {i}: columns of the {bad}"

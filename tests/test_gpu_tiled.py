@@ -149,10 +149,13 @@ def test_proj_f16_tt_adjacent_buffers(hip, rng):
 # number of blocks), each with a last batch block, output block and input step
 # that are only partly there: 1 (129 blocks of 32 x 128; an output count that
 # is no multiple of 4, one input step), 1 again (three input steps for two
-# groups of two), 2 (256 blocks of 64 x 128, 33 steps for four groups), 3 (320
-# blocks, odd steps), 4 (715 blocks); and fewer blocks than it takes.
+# groups of two, and 33: nine passes of the double-buffered loop), 2 (256 blocks
+# of 64 x 128, 33 steps for four groups), 3 (320 blocks, odd steps), 4 (715
+# blocks; two steps, and 33); 4096 or more inputs, where 2 stays up to 512 blocks
+# and 4 follows (260 and 585, 129 steps); and fewer blocks than it takes.
 @pytest.mark.parametrize("B,out_dim,in_dim", [(65, 5501, 32), (65, 5504, 96), (17, 16352, 64), (200, 8160, 1056),
-                                               (300, 8160, 160), (700, 8288, 64), (70, 1024, 96)])
+                                               (300, 8160, 160), (700, 8288, 64), (70, 1024, 96),
+                                               (65, 5504, 1056), (700, 8288, 1056), (256, 8320, 4128), (520, 8320, 4128)])
 def test_many_rows(hip, orc, rng, B, out_dim, in_dim):
     """Every epilogue and layout: within an fp16 ulp of the oracle, tiled
     layouts bit-identical to row-major, fp16 stores the fp32 ones narrowed."""
@@ -210,9 +213,11 @@ def test_many_rows(hip, orc, rng, B, out_dim, in_dim):
 
 
 # Stores of 8192 or more outputs, all of x in LDS: 64, 32 and 16 rows a
-# workgroup, with rows and outputs that are only partly there.
-@pytest.mark.parametrize("B,out_dim,in_dim", [(17, 8192, 256), (64, 8200, 1024), (30, 8208, 2048), (20, 8196, 4096)])
-def test_stores_through_lds(hip, orc, rng, B, out_dim, in_dim):
+# workgroup, with rows and outputs that are only partly there; and just past the
+# rows it holds, where the block-tiled kernel takes over in every layout.
+@pytest.mark.parametrize("B,out_dim,in_dim,gemm", [(17, 8192, 256, 0), (64, 8200, 1024, 0), (30, 8208, 2048, 0),
+                                                    (20, 8196, 4096, 0), (65, 8192, 1024, 1), (33, 16384, 4096, 1)])
+def test_stores_through_lds(hip, orc, rng, B, out_dim, in_dim, gemm):
     """Every layout with x in rows gives the same bits here too, in fp32 and
     fp16; x tiled takes the kernels that split the inputs over waves, whose sums
     run in another order: its fp16 stores are its fp32 ones, each checked."""
@@ -237,7 +242,7 @@ def test_stores_through_lds(hip, orc, rng, B, out_dim, in_dim):
     hip.proj_f16_tt(y[3], xt, wt, B, out_dim, in_dim, epilogue=hip.PROJ_STORE)
     check_projection(orc, x, w, host(y[0]).astype(np.float64))
     check_projection(orc, x, w, host(y[3]).astype(np.float64))
-    for i in (1, 2):
+    for i in (1, 2, 3) if gemm else (1, 2):
         assert_bitexact(host(y[i]), host(y[0]), f"layout {i}")
     h = [out(torch.int16) for _ in range(3)]
     hip.linear_f16(h[0], xr, dw)
