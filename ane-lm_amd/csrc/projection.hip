@@ -1150,6 +1150,14 @@ extern "C" int anelm_linear_f16(uint16_t* y16, const uint16_t* x16, const uint16
     hipStream_t st = as_stream(stream);
     if (lds_ok(a)) launch_lds<kStore16>(a, st);
     else if (mfma_ok(x16, true, w16, in_dim, ld_x) && rows_takes(a)) launch_rows<kXF16, kStore16>(a, st);
+    // Up to 512 tiles, 8 steps of loads in flight throughout: x16_mfma's shapes
+    // for longer sums and for 512 tiles were chosen on tiled weights (2560 x
+    // 4096, 32 rows: 19.5 us against 28.1; 4096 x 1024: 6.8 against 7.8); past
+    // that its 32 x 32 tiles win (4096 x 4096, 48 rows: 30.0 against 22.8).
+    // The same bits either way.
+    else if (mfma_ok(x16, true, w16, in_dim, ld_x) && !gemm_takes(a, kStore16) &&
+             (long)((out_dim + 15) / 16) * ((batch + 15) / 16) <= 512)
+        launch_mfma<true, 1, 1, 8, false, kStore16>(a, st);
     else if (mfma_ok(x16, true, w16, in_dim, ld_x)) x16_mfma<kStore16>(a, st);
     else launch_generic<true, kStore16>(a, st);
     return launch_status("linear_f16");
