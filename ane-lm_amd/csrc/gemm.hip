@@ -240,10 +240,14 @@ void launch_shape(const ProjArgs& a, hipStream_t st) {
 // row-major (the shape must not depend on the layout: the outputs of the
 // layouts are bit-identical).  nb32, nb64: blocks of 32 or 64 rows by 128
 // outputs.
-//   - Below 128 small blocks half the CUs idle and each pulls W through one
-//     CU's port: 64 rows of 1024 x 3072 down 8.1 us against 13.0; row-major 64
-//     rows of 4096 x 12288 down 64 against 109.  From 128: 100 rows of the
-//     latter 68 -> 41 tiled, 131 -> 111 row-major.
+//   - Up to 128 small blocks the other kernel's 16 or 32 row tiles are at most
+//     a workgroup per CU, here half the CUs idle and each pulls W through one
+//     CU's port: 64 rows of 1024 x 3072 down 8.1 us against 13.0; 500 rows of
+//     1024 x 3072 gate|up, 128 blocks, row-major 22.9 against 30.5, tiled 11 to
+//     33% slower at 4096 inputs.  Past 128 it loses nowhere in a sweep of 48
+//     to 1000 rows, 512 to 9728 inputs, each layout and epilogue (130 to 144
+//     blocks: 0.41 to 0.99 of its time).  Long sums without a SwiGLU win from
+//     128 on: 100 rows of 4096 x 12288 down 67 -> 64 tiled, 131 -> 116.
 //   - Up to one small block per CU nothing else fills the chip (140 rows of
 //     1024 x 3072 gate|up: 7.7 us, 64 x 128 blocks 9.5).
 //   - 64 x 128 in four groups up to one block per CU (2048 rows of 1024 x 3072
@@ -258,7 +262,8 @@ int gemm_shape(const ProjArgs& a, int epi) {
     const long cols = is_swiglu(epi) ? 2L * a.out_dim : a.out_dim;
     const long n128 = (cols + 127) / 128, K = a.in_dim;
     const long nb32 = (a.batch + 31) / 32 * n128, nb64 = (a.batch + 63) / 64 * n128;
-    if (a.batch <= 16 || nb32 < 128 || nb32 > (1L << 30)) return 0;   // (the launch's block count is an int)
+    if (a.batch <= 16 || nb32 < (K >= 8192 && !is_swiglu(epi) ? 128 : 129)) return 0;
+    if (nb32 > (1L << 30)) return 0;   // the launch's block count is an int
     if (nb32 <= 256) return 1;
     if (nb64 <= 256) return K >= 1024 ? 2 : 3;
     if (nb32 <= 512) return 1;

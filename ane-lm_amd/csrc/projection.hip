@@ -750,12 +750,14 @@ int cu_count() {
 // through the LDS kernel (measured for the 151936-row LM head; narrower W is
 // better served by more, smaller workgroups), as long as one workgroup's LDS
 // holds every row of x.  More rows mean reading W again per block of them, and
-// the block-tiled kernel wins: 151936 x 1024, 64 rows 60.9 us against 69.7 (its
+// with 128 blocks of 32 x 128 the block-tiled kernel (or, at 128 themselves,
+// proj_mfma_kernel) wins: 151936 x 1024, 64 rows 60.9 us against 69.7 (its
 // best shape), 100 rows 108 against 83; 151936 x 4096 (16 rows a workgroup), 48
 // rows 670 against 240.
 bool lds_ok(const ProjArgs& a) {
     return a.batch > 16 && a.out_dim >= 8192 && a.in_dim % 256 == 0 && a.in_dim <= 4096 && a.ld_x % 8 == 0 &&
-           aligned16(a.x) && aligned16(a.w) && (a.batch <= lds_rows(a.in_dim) || !gemm_takes(a, kStore));
+           aligned16(a.x) && aligned16(a.w) &&
+           (a.batch <= lds_rows(a.in_dim) || (a.batch + 31L) / 32 * ((a.out_dim + 127L) / 128) < 128);
 }
 
 template <int EPI, bool TILED = false>

@@ -152,10 +152,12 @@ def test_proj_f16_tt_adjacent_buffers(hip, rng):
 # groups of two, and 33: nine passes of the double-buffered loop), 2 (256 blocks
 # of 64 x 128, 33 steps for four groups), 3 (320 blocks, odd steps), 4 (715
 # blocks; two steps, and 33); 4096 or more inputs, where 2 stays up to 512 blocks
-# and 4 follows (260 and 585, 129 steps); and fewer blocks than it takes.
+# and 4 follows (260 and 585, 129 steps); and fewer blocks than it takes: 24,
+# and 128, which it takes from 8192 inputs.
 @pytest.mark.parametrize("B,out_dim,in_dim", [(65, 5501, 32), (65, 5504, 96), (17, 16352, 64), (200, 8160, 1056),
                                                (300, 8160, 160), (700, 8288, 64), (70, 1024, 96),
-                                               (65, 5504, 1056), (700, 8288, 1056), (256, 8320, 4128), (520, 8320, 4128)])
+                                               (65, 5504, 1056), (700, 8288, 1056), (256, 8320, 4128), (520, 8320, 4128),
+                                               (100, 4096, 96), (100, 4084, 8192)])
 def test_many_rows(hip, orc, rng, B, out_dim, in_dim):
     """Every epilogue and layout: within an fp16 ulp of the oracle, tiled
     layouts bit-identical to row-major, fp16 stores the fp32 ones narrowed."""
@@ -214,9 +216,11 @@ def test_many_rows(hip, orc, rng, B, out_dim, in_dim):
 
 # Stores of 8192 or more outputs, all of x in LDS: 64, 32 and 16 rows a
 # workgroup, with rows and outputs that are only partly there; and just past the
-# rows it holds, where the block-tiled kernel takes over in every layout.
+# rows it holds, where the block-tiled kernel takes over in every layout (and
+# proj_mfma_kernel at 128 blocks).
 @pytest.mark.parametrize("B,out_dim,in_dim,gemm", [(17, 8192, 256, 0), (64, 8200, 1024, 0), (30, 8208, 2048, 0),
-                                                    (20, 8196, 4096, 0), (65, 8192, 1024, 1), (33, 16384, 4096, 1)])
+                                                    (20, 8196, 4096, 0), (65, 8192, 1024, 1), (33, 16384, 4096, 1),
+                                                    (33, 8192, 2048, 1)])
 def test_stores_through_lds(hip, orc, rng, B, out_dim, in_dim, gemm):
     """Every layout with x in rows gives the same bits here too, in fp32 and
     fp16; x tiled takes the kernels that split the inputs over waves, whose sums
