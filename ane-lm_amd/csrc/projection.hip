@@ -665,15 +665,28 @@ void proj_dot(const ProjArgs& a, hipStream_t st) {
     else dot_shape<8, XM, EPI>(a, st);
 }
 
-// Where the dot kernel beats the MFMA kernels: one or two rows of x (gate|up
-// of 2560 x 9728, 2 rows: 19.1 us against 24.1 in rows.hip), but, without a
-// norm or a SwiGLU (plain), not two rows of 4096 or more inputs into 2560 or more outputs, which it takes in
-// several rounds of loads (2560 x 9728 down: 15.1 against 12.3); and up to
-// eight for narrow out_dim and short rows (3 rows, 1024 x 2048: 3.5 against
-// 3.9; 5 rows, 896 x 4864: 8.3 against 5.8).
-bool dot_wins(long batch, int out_dim, int in_dim, bool plain) {
-    if (batch == 2 && plain && in_dim >= 4096 && out_dim >= 2560) return false;
-    return batch <= 2 || (batch <= 8 && out_dim <= 1024 && in_dim <= 3072);
+// Where the dot kernel beats the MFMA kernels (rows.hip up to 16 rows).  It
+// takes a row of x in rounds of up to 3072 inputs and one more for what is
+// left, so rows of whole rounds suit it.  The choice must not depend on the
+// form of x: fp32 rows that are fp16 values and the fp16 rows themselves give
+// the same bits.  us, dot / rows.hip, fp16 x unless said:
+//   One row always; two with a norm (2560 x 9728 gate|up: 19.1 / 24.1) or a
+//   SwiGLU.  Two rows plain: to 2560 or more outputs from 4096 or more inputs
+//   rows.hip wins (2560 x 4096 0.73 of dot's time, 4096 x 9728 0.76, 8192 x
+//   4864 0.82; fp32 rows 0.50-0.55), but not whole rounds into half as many
+//   outputs or more (8192 x 6144 19.4 / 21.9, 4096 x 6144 11.0 / 11.7; 4096 x
+//   12288, below that line, 0.92).
+//   Up to eight rows into 1024 or fewer outputs: rows of one round (3 rows,
+//   1024 x 2048: 3.5 / 3.9).  Past that rows.hip takes them (5 rows, 896 x 4864
+//   8.3 / 5.8), but three and four rows stay for a norm (4 rows, 512 gate|up
+//   pairs x 4096 7.7 / 9.2) and for whole rounds (512 pairs x 6144, SwiGLU 6.7
+//   / 8.1, 512 x 6144 add 5.2 / 5.9; fp32 rows lose there, 1.6-2 of rows.hip's).
+bool dot_wins(long batch, int out_dim, int in_dim, bool norm, bool swiglu) {
+    const bool whole = in_dim % 3072 == 0;
+    if (batch == 2 && !norm && !swiglu && in_dim >= 4096 && out_dim >= 2560) return whole && out_dim >= in_dim / 2;
+    if (batch <= 2) return true;
+    if (batch > 8 || out_dim > 1024) return false;
+    return in_dim <= 3072 || (batch <= 4 && (norm || whole));
 }
 
 // y and x must not share memory: workgroups write y while others still read x.
@@ -858,7 +871,7 @@ extern "C" int anelm_proj_f16(float* y, const float* x, const uint16_t* w16, lon
     hipStream_t st = as_stream(stream);
     const ProjArgs a = args(y, x, w16, batch, out_dim, in_dim, ld_x, ld_y);
     const bool dot = dot_ok(x, w16, batch, in_dim, ld_x);
-    if (mfma_ok(x, false, w16, in_dim, ld_x) && !(dot && dot_wins(batch, out_dim, in_dim, true))) return proj_mfma<false>(a, st);
+    if (mfma_ok(x, false, w16, in_dim, ld_x) && !(dot && dot_wins(batch, out_dim, in_dim, false, false))) return proj_mfma<false>(a, st);
     if (dot) {
         proj_dot<kXF32, kStore>(a, st);
     } else {
@@ -934,7 +947,7 @@ void x16_mfma(const ProjArgs& a, hipStream_t st) {
 
 template <int EPI>
 void x16_fused(const ProjArgs& a, hipStream_t st) {
-    if (dot16_ok(static_cast<const uint16_t*>(a.x), a.w, a.batch, a.in_dim, a.ld_x) && dot_wins(a.batch, a.out_dim, a.in_dim, !is_swiglu(EPI)))
+    if (dot16_ok(static_cast<const uint16_t*>(a.x), a.w, a.batch, a.in_dim, a.ld_x) && dot_wins(a.batch, a.out_dim, a.in_dim, false, is_swiglu(EPI)))
         proj_dot<kXF16, EPI>(a, st);
     else if (rows_takes(a)) launch_rows<kXF16, EPI>(a, st);
     else if (EPI == kStore && lds_ok(a)) launch_lds<kStore>(a, st);
@@ -1094,8 +1107,8 @@ extern "C" int anelm_proj_f16_fused(void* y, const float* x, const uint16_t* w16
     a.pair_rows = out_dim;  // SwiGLU: W holds out_dim gate rows, then out_dim up rows
     hipStream_t st = as_stream(stream);
     const bool norm = norm_bf16 != nullptr;
-    const bool plain = !norm && epilogue <= ANELM_PROJ_ADD;
-    if (dot_ok(x, w16, batch, in_dim, ld_x) && dot_wins(batch, out_dim, in_dim, plain) && (!norm || in_dim <= kDotNormMaxIn)) {
+    const bool swiglu = epilogue >= ANELM_PROJ_SWIGLU;
+    if (dot_ok(x, w16, batch, in_dim, ld_x) && dot_wins(batch, out_dim, in_dim, norm, swiglu) && (!norm || in_dim <= kDotNormMaxIn)) {
         switch (epilogue) {
             case ANELM_PROJ_STORE:
                 if (norm) proj_dot<kXNorm, kStore>(a, st);

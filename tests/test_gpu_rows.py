@@ -14,9 +14,11 @@ pytestmark = pytest.mark.gpu
 # last chunk that is partly there, more chunks than waves; fewer than 16
 # outputs, a ragged last tile, both wave counts (8192 outputs either side); the
 # smallest and largest row counts of each staging size; two rows where the dot
-# kernel hands over.
+# kernel hands over; and where it keeps two to four rows of whole rounds of its
+# loads, or with a norm.
 @pytest.mark.parametrize("B,out_dim,in_dim", [(3, 10, 32), (4, 8208, 160), (5, 33, 96), (8, 1040, 4128), (9, 16, 1056),
-                                               (16, 8191, 64), (6, 8192, 256), (13, 2048, 2080), (2, 2576, 4096)])
+                                               (16, 8191, 64), (6, 8192, 256), (13, 2048, 2080), (2, 2576, 4096),
+                                               (2, 3080, 6144), (4, 520, 6144), (3, 1024, 4096)])
 def test_few_rows(hip, orc, rng, B, out_dim, in_dim):
     import torch
 
