@@ -168,7 +168,7 @@ __device__ __forceinline__ float ld_dev(const float* p) {
 template <int D>
 __device__ void merge_head(const AttnArgs& a, long b, int h, int lane, int live) {
     // Chunks whose partials are in flight at once: 32 held 64 more registers
-    // through the whole kernel (3 waves per SIMD instead of 5) for a merge that
+    // through the whole kernel (3 waves per SIMD instead of 4) for a merge that
     // ring_chunk keeps to a few batches (16 x 1024 ragged rows 26.9 -> 24.6 us).
     constexpr int kBatch = 8;
     const int ns = a.nsplit;

@@ -45,9 +45,9 @@ __device__ __forceinline__ uint32_t f16_bits_rne(float v) {
 // one contiguous 1 KB piece), the input layout of the tiled projection.  A row
 // writes 16 bytes of each 128-byte line there and seven neighbours the rest,
 // so rows in launch order, dealt to the 8 XCDs in turn, sent every line to
-// memory in eight parts.  In a grid of whole 64s, workgroup i takes row
-// 8 * (i % 8) + (i / 8) % 8 of its 64, so each XCD's L2 gathers whole lines:
-// 2048 x 4096 21.5 -> 15.2 us, 500 x 2560 5.2 -> 4.0, 300 x 1024 2.5 -> 2.2.
+// memory in eight parts.  From 128 rows, in a grid of whole 64s, workgroup i
+// takes row 8 * (i % 8) + (i / 8) % 8 of its 64, so each XCD's L2 gathers whole
+// lines: 2048 x 4096 21.5 -> 15.2 us, 500 x 2560 5.2 -> 4.0, 300 x 1024 2.5 -> 2.2.
 template <int NV, int DT, bool ADD, bool O16 = false, bool FULL = false, bool TILE = false>
 __global__ __launch_bounds__(1024) void rmsnorm_row_kernel(void* out, float* x, const float* y,
                                                            const void* w, long rows, int dim,
@@ -181,9 +181,14 @@ static int launch_rmsnorm_dt(void* out, float* x, const float* y, const void* w,
     if (vec && nvec <= 1024 * 4) {
         int nv, threads;
         rms_row_geometry(rows, nvec, nv, threads);
-        // Whole 64s for the tiled rows' order: not below 128 rows (a decode step
-        // of 64 sequences took 1.107 ms without it, 1.109 with), nor past 2^24
-        // rows, where rounding up could pass the grid's limit.
+        // Whole 64s for the tiled rows' order, from 128 rows: 2560 and 4096 wide
+        // it wins by 13 to 24% from there on (128 x 2560 2.95 -> 2.31 us), but loses
+        // up to 11% below (48 x 2560 2.37 -> 2.65).  1024 wide it loses alone up to
+        // 200 rows (128: 2.17 -> 2.42 us), yet the projection after it then reads
+        // whole lines: a decode step of 128 sequences 1.538 -> 1.527 ms.  At 64
+        // sequences the step does not tell the two apart (1.139 to 1.143 ms and
+        // 1.134 to 1.145 over three runs each).  Not past 2^24 rows, where rounding
+        // up could pass the grid's limit.
         const dim3 grd((unsigned)(TILE && rows >= 128 && rows <= (1L << 24) ? (rows + 63) / 64 * 64 : rows));
         const bool full = nvec == nv * threads;
 #define ANELM_RMS_ROW(NV_, FULL_) \

@@ -1174,7 +1174,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 8 ? 5 
     // stage 1: the chunk maximum of the adjusted logits
     // A whole chunk, every chunk of a row but its last, takes no selects here
     // and in the exponentials: 64 rows of 151936, 63.2 -> 60.2 us per call
-    // (the stages are bound by their vector instructions).
+    // (vector instructions are about half of the stages' time).
     float best = -INFINITY;
     if (nvalid == kCH) {
 #pragma unroll
