@@ -649,8 +649,9 @@ int plan(AttnArgs& a, long batch, int D, int bound, void* ws, size_t ws_bytes) {
     // rings that one workgroup can do need no workspace: without one, it does them
     if (bound <= kMaxChunk && !serves(a.nsplit)) a.nsplit = 1;
     // Eight waves take a chunk in half the rounds of loads of four (64
-    // sequences of ragged lengths up to 2048 rows 109 us against 128, though
-    // all 2048 long 171.5 against 169.8; 1 x 512 rows 7.8 against 8.4); four where
+    // sequences of ragged lengths up to 2048 rows 109 us against 128; 1 x 512
+    // rows 7.8 against 8.4), though 64 rings of 1024 rows and two q heads each,
+    // all equally long, take 86.0 us against 85.3; four where
     // every ring is a round or two and the pairs fill the chip anyway (64
     // sequences x 128 rows: 13.8 against 14.3).  With more than four q heads
     // (158 VGPRs, three waves per SIMD) a CU holds one workgroup of eight waves
