@@ -319,9 +319,11 @@ def test_bounded_launch_ring_past_bound(hip, orc, rng):
 
 
 def test_workspace_size_covers_smaller_batches(hip):
-    """The size for a batch serves every smaller batch: the chunk grows with
-    the batch, so a smaller batch can need more partials (three sequences at
-    capacity 32768 need more than four)."""
+    """The size for a batch serves every smaller batch: the chunk it counts
+    grows with the batch, so a smaller batch can be counted for more partials
+    (three sequences at capacity 32768 for more than four).  The call itself
+    launches fewer; the CPU sweep of the plan and test_workspace_filled are
+    what come near the size."""
     import torch
 
     nq, nk, D, cap = 32, 8, 128, 32768
