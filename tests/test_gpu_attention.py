@@ -349,11 +349,12 @@ def test_workspace_size_covers_smaller_batches(hip):
 # heads with eight waves and with four.
 @pytest.mark.parametrize("B,nq,nk,cap,lens", [
     (12, 16, 8, 512, [0, 1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 512]),
-    (3, 8, 4, 1100, [1100, 897, 340]), (8, 8, 8, 1024, [1024, 129, 255, 256, 257, 384, 385, 640]),
+    (2, 8, 4, 1100, [1100, 897]), (3, 8, 4, 1100, [1100, 897, 340]), (8, 8, 8, 1024, [1024, 129, 255, 256, 257, 384, 385, 640]),
     (1, 8, 8, 8192, [500]), (2, 8, 4, 1100, [1024, 1025]),
     (6, 16, 8, 2048, [341, 342, 1562, 1563, 2048, 256]), (16, 20, 4, 256, [256, 1, 33, 65, 128, 129, 192, 193] * 2),
     (32, 8, 4, 600, [128, 129, 256, 257, 512, 513, 585, 586] * 4), (33, 8, 4, 256, [256, 129, 128] * 11),
-    (33, 8, 4, 300, [255, 256, 257] * 11), (40, 8, 8, 1000, [1000, 512, 513, 687, 688] * 8),
+    (33, 8, 4, 300, [255, 256, 257] * 11), (40, 8, 8, 1000, [1000, 512, 513, 300] * 10),
+    (40, 8, 8, 1000, [1000, 512, 513, 687, 688] * 8),
     (64, 4, 4, 128, [128, 1, 31, 32, 33, 64, 65, 127] * 8),
     (3, 16, 2, 400, [400, 129, 64]), (20, 16, 2, 1100, [1100, 614, 128, 129, 900] * 4)])
 def test_chunk_and_batch_edges(hip, orc, rng, B, nq, nk, cap, lens):
